@@ -509,13 +509,19 @@ msfec_status msfec_rt_destroy(msfec_rt_handle h);
 typedef struct {
   int n_refine_local; /* l, 1..4                                                      */
   int flags;          /* MSFEC_FLAG_*                                                 */
-  int solver;         /* 0: the dense direct solve for l <= 2 (the interior system of
-                         up to 256 unknowns factored on the matrix cores) and MINRES
-                         above; MSFEC_SOLVER_CG: matrix-free MINRES for every l      */
-  int max_iter;       /* MINRES iteration limit, 0: 20000; a solve that reaches it
-                         flags its cell MSFEC_CELL_NOT_CONVERGED                      */
-  double rtol;        /* MINRES stop: preconditioned residual <= rtol x the initial
-                         one, 0: 1e-14                                                */
+  int solver;         /* 0: without a reaction term, the discrete exact sequence (one
+                         scalar problem per edge basis, eliminated for l <= 2 and
+                         solved by conjugate gradients above, and trigonometric
+                         transforms) for the cells with A^-1 positive definite and
+                         B > 0 at every Gauss point; otherwise the dense direct solve
+                         for l <= 2 (the interior system of up to 256 unknowns
+                         factored on the matrix cores) and MINRES above;
+                         MSFEC_SOLVER_CG: matrix-free MINRES for every l             */
+  int max_iter;       /* iteration limit (MINRES, conjugate gradients), 0: 20000; a
+                         solve that reaches it flags its cell
+                         MSFEC_CELL_NOT_CONVERGED                                     */
+  double rtol;        /* stop: preconditioned residual (MINRES) or residual (CG) <=
+                         rtol x the initial one, 0: 1e-14                             */
 } msfec_nrt_params;
 
 typedef struct msfec_nrt_batch *msfec_nrt_handle;
@@ -570,7 +576,9 @@ msfec_status msfec_nrt_reconstruct(msfec_nrt_handle h, const double *w, int w_lo
  * solve reached max_iter, MSFEC_CELL_NONFINITE for non-finite data. */
 msfec_status msfec_nrt_get_cell_status(msfec_nrt_handle h, int *status);
 
-/* MINRES iterations of the last compute, n_cells x 18 ints on the host (the
+/* Iterations of the last compute, n_cells x 18 ints on the host: of MINRES, or
+ * for a cell solved by the exact sequence of the conjugate gradients of the
+ * edge bases (0 for the face bases) (the
  * reference's solver_control.last_step() of solve_iterative,
  * ned_rt_basis.cc:796-801); MSFEC_ERR_STATE for a handle on the dense path.
  * Synchronizes. */

@@ -54,6 +54,7 @@
 #include <vector>
 
 #include "msfec.h"
+#include "msfec_nrt_seq.hpp"
 
 namespace msfec_detail {
 extern thread_local std::string g_last_error;
@@ -283,6 +284,7 @@ struct NrtArgs {
   double* b;            // n_cells x 18
   int* status;          // n_cells
   int N;
+  const int* need;  // n_cells, or null: only the cells flagged here are computed
 };
 
 // entry (a, b) of the local matrix of fine cell c: K' (face rows negated,
@@ -358,6 +360,7 @@ __global__ __launch_bounds__(Nd<L>::NT) void nrt_basis_kernel(NrtArgs g) {
   extern __shared__ double sm[];
   __shared__ int s_flag;
   const int cell = blockIdx.x, tid = threadIdx.x;
+  if (g.need && !g.need[cell]) return;
   const int lane = tid & 63, w = tid >> 6, ll = lane & 15, lh = lane >> 4;
   const int N = g.N;
 
@@ -1001,6 +1004,7 @@ struct NrtItArgs {
   int* its;          // n_cells x 18: MINRES iterations
   int* flg;          // n_cells x 18: MSFEC_CELL_* of every solve
   int* status;       // n_cells
+  const int* need;   // n_cells, or null: only the cells flagged here are computed
   int n_cells, N, n, max_iter;
   double rtol;
 };
@@ -1213,6 +1217,7 @@ __global__ __launch_bounds__(256) void nrt_it_local_kernel(NrtItArgs g) {
   __shared__ double Wt[78 * 8], PP[21 * 8], DD[21];
   __shared__ int cmp[78];
   const int cell = blockIdx.x, tid = threadIdx.x;
+  if (g.need && !g.need[cell]) return;
   V3 Hc, h;
   it_sizes(g.verts + (size_t)cell * 24, Hc, h, M);
   const double w8 = h.x * h.y * h.z * 0.125;
@@ -1306,6 +1311,7 @@ template <int L>
 __global__ __launch_bounds__(256) void nrt_it_diag_kernel(NrtItArgs g) {
   constexpr int M = 1 << L, nfc = M * M * M;
   const int cell = blockIdx.x;
+  if (g.need && !g.need[cell]) return;
   const double* lm = g.LM + (size_t)cell * kLM * nfc;
   const double* Cc = g.CC + (size_t)cell * 72;
   double* pd = g.PD + (size_t)cell * g.N;
@@ -1424,6 +1430,7 @@ __global__ __launch_bounds__(256) void nrt_it_coarse_kernel(NrtItArgs g) {
   typedef ItCoarse<M> CS;
   extern __shared__ double uf[];  // NF
   const int cell = blockIdx.x / CS::NC, J = blockIdx.x % CS::NC, tid = threadIdx.x;
+  if (g.need && !g.need[cell]) return;
   const double* lm = g.LM + (size_t)cell * kLM * nfc;
   const double* Cc = g.CC + (size_t)cell * 72;
   // the cells with a face in J, widened by the reach of C diag(Me)^-1 C^T
@@ -1494,6 +1501,7 @@ __global__ __launch_bounds__(64) void nrt_it_edgeas_kernel(NrtItArgs g) {
   __shared__ double A[64][145];
   const int tid = threadIdx.x;
   const int cell = blockIdx.x / (nfc / CPB), c = (blockIdx.x % (nfc / CPB)) * CPB + tid;
+  if (g.need && !g.need[cell]) return;
   if (tid >= CPB) return;
   const int c0 = c % M, c1 = (c / M) % M, c2 = c / (M * M);
   const int sc = it_lmc<M>(c0, c1, c2);
@@ -1558,6 +1566,7 @@ template <int L>
 __global__ __launch_bounds__(1024) void nrt_it_coarse_inv_kernel(NrtItArgs g) {
   constexpr int M = 1 << L;
   constexpr int NC = ItCoarse<M>::NC;
+  if (g.need && !g.need[blockIdx.x]) return;
   double* A = g.S0 + (size_t)blockIdx.x * NC * NC;
   for (int k = 0; k < NC; ++k) {
     const double p = 1.0 / A[k * NC + k];
@@ -1642,7 +1651,7 @@ __global__ __launch_bounds__(kItNT) void nrt_minres_kernel(NrtItArgs g) {
   __shared__ double sq[NC], scq[NC];
   const int bid = blockIdx.x, slot = bid >> 3;
   const int cell = (slot / kNB) * 8 + (bid & 7), r = slot % kNB;
-  if (cell >= g.n_cells) return;
+  if (cell >= g.n_cells || (g.need && !g.need[cell])) return;
   const int tid = threadIdx.x, N = g.N, n = g.n;
   V3 Hc, h;
   it_sizes(g.verts + (size_t)cell * 24, Hc, h, M);
@@ -1833,6 +1842,7 @@ __global__ __launch_bounds__(256) void nrt_it_element_kernel(NrtItArgs g) {
   constexpr int nx = M * (M + 1) * (M + 1), ne = 3 * nx;
   __shared__ double red[4][kNB + 1];
   const int cell = blockIdx.x / kNB, i = blockIdx.x % kNB, tid = threadIdx.x;
+  if (g.need && !g.need[cell]) return;
   const int N = g.N;
   const double* xi = g.X + ((size_t)cell * kNB + i) * N;
   const double* fl = g.FL + (size_t)cell * nfc * 6;
@@ -1874,7 +1884,7 @@ __global__ __launch_bounds__(256) void nrt_it_element_kernel(NrtItArgs g) {
 // Per-cell status from the 18 solves and the element matrix.
 __global__ __launch_bounds__(256) void nrt_it_status_kernel(NrtItArgs g) {
   const int cell = blockIdx.x * 256 + threadIdx.x;
-  if (cell >= g.n_cells) return;
+  if (cell >= g.n_cells || (g.need && !g.need[cell])) return;
   int st = MSFEC_CELL_OK;
   for (int r = 0; r < kNB; ++r) {
     const int f = g.flg[(size_t)cell * kNB + r];
@@ -2488,6 +2498,8 @@ struct msfec_nrt_batch {
   double* d_S0 = nullptr;
   int* d_agg = nullptr;
   double* d_EI = nullptr;
+  // the bases by the exact sequence (solver 0 without a reaction term)
+  double* d_seq = nullptr;  // one allocation: weights, rows, right-hand sides, potentials, ints
   bool coef_set = false, has_r = false, has_f = false, computed = false;
   hipStream_t stream = nullptr;
   // per timed compute: start, after the local matrices and preconditioner,
@@ -2508,7 +2520,8 @@ void nrt_free(msfec_nrt_batch* h) {
   void* ptrs[] = {h->d_verts, h->d_ainv, h->d_b,  h->d_r,   h->d_f,  h->d_icell, h->d_cdof,
                   h->d_f2i,   h->d_amap, h->d_tnz, h->d_X,  h->d_M,  h->d_rhs,   h->d_w,
                   h->d_status, h->d_idof, h->d_LM, h->d_CC, h->d_FL, h->d_PD,    h->d_WK,
-                  h->d_its,   h->d_flg,  h->d_S0, h->d_agg, h->d_EI};
+                  h->d_its,   h->d_flg,  h->d_S0, h->d_agg, h->d_EI,
+                  h->d_seq};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (auto& set : h->ev_sets)
@@ -2535,7 +2548,7 @@ msfec_status nrt_out(hipStream_t s, double* dst, const double* src, size_t count
 }
 
 template <int L>
-msfec_status nrt_launch(msfec_nrt_batch* h, hipStream_t s) {
+msfec_status nrt_launch(msfec_nrt_batch* h, hipStream_t s, const int* need) {
   typedef Nd<L> D;
   const size_t lds = (size_t)D::total * sizeof(double);
   NRT_HIP(hipFuncSetAttribute((const void*)nrt_basis_kernel<L>,
@@ -2556,13 +2569,15 @@ msfec_status nrt_launch(msfec_nrt_batch* h, hipStream_t s) {
   a.b = h->d_rhs;
   a.status = h->d_status;
   a.N = h->tab.N;
+  a.need = need;
   hipLaunchKernelGGL(nrt_basis_kernel<L>, dim3(h->n_cells), dim3(D::NT), lds, s, a);
   NRT_HIP(hipGetLastError());
   return MSFEC_OK;
 }
 
 template <int L>
-msfec_status nrt_it_launch(msfec_nrt_batch* h, hipStream_t s, std::array<hipEvent_t, 4>* ev) {
+msfec_status nrt_it_launch(msfec_nrt_batch* h, hipStream_t s, std::array<hipEvent_t, 4>* ev,
+                           const int* need) {
   NrtItArgs a{};
   a.verts = h->d_verts;
   a.ainv = h->d_ainv;
@@ -2584,6 +2599,7 @@ msfec_status nrt_it_launch(msfec_nrt_batch* h, hipStream_t s, std::array<hipEven
   a.agg = h->d_agg;
   a.EI = h->d_EI;
   a.status = h->d_status;
+  a.need = need;
   a.n_cells = h->n_cells;
   a.N = h->tab.N;
   a.n = h->tab.n;
@@ -2732,7 +2748,12 @@ msfec_status msfec_nrt_create(const msfec_nrt_params* params, int n_cells, const
     NRT_TRY(nrt_alloc(&h->d_agg, agg.size()));
     NRT_TRY(nrt_in(h->stream, h->d_agg, agg.data(), agg.size() * sizeof(int), MSFEC_HOST));
     NRT_TRY(nrt_alloc(&h->d_S0, nc * NC * NC));
-  } else {
+  }
+  if (params->solver == 0) {
+    // 51 doubles per fine cell, the sums of the weights and 25 ints per cell
+    NRT_TRY(nrt_alloc(&h->d_seq, nc * (51 * nfc + nfc + 1) + (nc * 25 + 1) / 2));
+  }
+  if (!h->iter) {
     std::vector<unsigned short> amap;
     std::vector<unsigned char> tnz;
     if (l == 1) nrt_amap<1>(h->tab, amap, tnz);
@@ -2778,24 +2799,55 @@ msfec_status msfec_nrt_compute(msfec_nrt_handle h, void* stream) {
     ev = &h->ev_sets[h->ev_used++];
     NRT_HIP(hipEventRecord((*ev)[0], s));
   }
+  std::array<hipEvent_t, 4>* const set = ev;
   msfec_status st;
+  // Without a reaction term the exact sequence gives the bases; the general
+  // solver then takes the cells that it flags (an indefinite A^-1, B <= 0,
+  // data that are not finite) and its workgroups leave the others at once.
+  // An explicit MSFEC_SOLVER_CG asks for MINRES.
+  const int* need = nullptr;
+  if (h->d_seq && !h->has_r) {
+    const size_t nc = (size_t)h->n_cells, nfc = (size_t)1 << (3 * h->l);
+    msfec_detail::NrtSeq q{};
+    q.verts = h->d_verts;
+    q.ainv = h->d_ainv;
+    q.bq = h->d_b;
+    q.fq = h->has_f ? h->d_f : nullptr;
+    q.st = h->d_seq;
+    q.rhs = q.st + nc * 27 * nfc;
+    q.phi = q.rhs + nc * 12 * nfc;
+    q.W = q.phi + nc * 12 * nfc;
+    q.iters = reinterpret_cast<int*>(q.W + nc * (nfc + 1));
+    q.general = q.iters + nc * 24;
+    q.X = h->d_X;
+    q.Mat = h->d_M;
+    q.b = h->d_rhs;
+    q.status = h->d_status;
+    q.its = h->d_its;
+    q.n_cells = h->n_cells;
+    q.max_iter = h->prm.max_iter > 0 ? h->prm.max_iter : 20000;
+    q.rtol = h->prm.rtol > 0.0 ? h->prm.rtol : 1e-14;
+    NRT_HIP(msfec_detail::nrt_seq(h->l, q, s, ev && h->iter ? &(*ev)[1] : nullptr));
+    need = q.general;
+    if (h->iter) ev = nullptr;  // its two inner events are recorded
+  }
   if (h->iter) {
     switch (h->l) {
-      case 1: st = nrt_it_launch<1>(h, s, ev); break;
-      case 2: st = nrt_it_launch<2>(h, s, ev); break;
-      case 3: st = nrt_it_launch<3>(h, s, ev); break;
-      default: st = nrt_it_launch<4>(h, s, ev); break;
+      case 1: st = nrt_it_launch<1>(h, s, ev, need); break;
+      case 2: st = nrt_it_launch<2>(h, s, ev, need); break;
+      case 3: st = nrt_it_launch<3>(h, s, ev, need); break;
+      default: st = nrt_it_launch<4>(h, s, ev, need); break;
     }
   } else {
-    st = h->l == 1 ? nrt_launch<1>(h, s) : nrt_launch<2>(h, s);
+    st = h->l == 1 ? nrt_launch<1>(h, s, need) : nrt_launch<2>(h, s, need);
   }
   if (st != MSFEC_OK) return st;
-  if (ev) {
+  if (set) {
     if (!h->iter) {
-      NRT_HIP(hipEventRecord((*ev)[1], s));
-      NRT_HIP(hipEventRecord((*ev)[2], s));
+      NRT_HIP(hipEventRecord((*set)[1], s));
+      NRT_HIP(hipEventRecord((*set)[2], s));
     }
-    NRT_HIP(hipEventRecord((*ev)[3], s));
+    NRT_HIP(hipEventRecord((*set)[3], s));
   }
   h->computed = true;
   return MSFEC_OK;

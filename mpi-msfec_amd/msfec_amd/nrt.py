@@ -28,8 +28,10 @@ def nrt_sizes(n_refine_local):
 class NedRTBasisBatch:
     def __init__(self, vertices, n_refine_local=2, timing=False, solver=0, max_iter=0, rtol=0.0):
         """vertices: n_cells x 8 x 3, axis-aligned boxes in deal.II vertex order.
-        solver 0: the dense direct solve for l <= 2, MINRES above;
-        SOLVER_CG: MINRES at every l (max_iter 0: 20000, rtol 0: 1e-14)."""
+        solver 0: without a reaction term the exact sequence (scalar problems
+        and trigonometric transforms), with one the dense direct solve for
+        l <= 2 and MINRES above; SOLVER_CG: MINRES at every l (max_iter 0:
+        20000, rtol 0: 1e-14)."""
         self._lib = L.load()
         self._h = ctypes.c_void_p()
         p = L.NrtParams()
@@ -118,7 +120,7 @@ class NedRTBasisBatch:
         return st
 
     def get_iterations(self):
-        """MINRES iterations of every basis solve, n_cells x 18 (MINRES path only)."""
+        """Iterations of every basis solve, n_cells x 18 (l > 2 or SOLVER_CG)."""
         its = np.empty((self.n_cells, 18), dtype=np.int32)
         L.check(self._lib.msfec_nrt_get_iterations(
             self._h, its.ctypes.data_as(ctypes.POINTER(ctypes.c_int))))
