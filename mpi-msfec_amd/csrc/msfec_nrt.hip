@@ -2750,8 +2750,8 @@ msfec_status msfec_nrt_create(const msfec_nrt_params* params, int n_cells, const
     NRT_TRY(nrt_alloc(&h->d_S0, nc * NC * NC));
   }
   if (params->solver == 0) {
-    // 51 doubles per fine cell, the sums of the weights and 25 ints per cell
-    NRT_TRY(nrt_alloc(&h->d_seq, nc * (51 * nfc + nfc + 1) + (nc * 25 + 1) / 2));
+    // 39 doubles per fine cell, the sums of the weights and 25 ints per cell
+    NRT_TRY(nrt_alloc(&h->d_seq, nc * (39 * nfc + nfc + 1) + (nc * 25 + 1) / 2));
   }
   if (!h->iter) {
     std::vector<unsigned short> amap;
@@ -2814,7 +2814,7 @@ msfec_status msfec_nrt_compute(msfec_nrt_handle h, void* stream) {
     q.bq = h->d_b;
     q.fq = h->has_f ? h->d_f : nullptr;
     q.st = h->d_seq;
-    q.rhs = q.st + nc * 27 * nfc;
+    q.rhs = q.st + nc * 15 * nfc;
     q.phi = q.rhs + nc * 12 * nfc;
     q.W = q.phi + nc * 12 * nfc;
     q.iters = reinterpret_cast<int*>(q.W + nc * (nfc + 1));

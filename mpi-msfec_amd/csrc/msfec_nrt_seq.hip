@@ -34,10 +34,13 @@
 
 #include "msfec.h"
 #include "msfec_q1t.hpp"
+#include "msfec_wave.hpp"
 
 namespace {
 
 using msfec_detail::NrtSeq;
+using msfec_wave::block_sums;
+using msfec_wave::wave_sum;
 
 constexpr double kGp[2] = {0.21132486540518711775, 0.78867513459481288225};
 constexpr int kLnAx[12] = {1, 1, 0, 0, 1, 1, 0, 0, 2, 2, 2, 2};
@@ -143,43 +146,6 @@ struct Seq {
   static constexpr int NW = NT / 64;
 };
 
-__device__ __forceinline__ double wsum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
-
-// Block sums of 16 values per thread; thread t < 16 returns the t-th.  A wave
-// sums them by halving: lanes 32, 16, 8 and 4 apart exchange half of what
-// they hold (15 exchanges, not 96), then the 4 lanes left with the same value
-// add up.
-template <int NW>
-__device__ __forceinline__ double block_sums(const double* v, double (*red)[16]) {
-  const int lane = threadIdx.x & 63;
-  double a[8];
-  int hi = lane >> 5 & 1;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) a[k] = (hi ? v[8 + k] : v[k]) + __shfl_xor(hi ? v[k] : v[8 + k], 32);
-  hi = lane >> 4 & 1;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) a[k] = (hi ? a[4 + k] : a[k]) + __shfl_xor(hi ? a[k] : a[4 + k], 16);
-  hi = lane >> 3 & 1;
-#pragma unroll
-  for (int k = 0; k < 2; ++k) a[k] = (hi ? a[2 + k] : a[k]) + __shfl_xor(hi ? a[k] : a[2 + k], 8);
-  hi = lane >> 2 & 1;
-  double s = (hi ? a[1] : a[0]) + __shfl_xor(hi ? a[0] : a[1], 4);
-  s += __shfl_xor(s, 2);
-  s += __shfl_xor(s, 1);
-  __syncthreads();
-  if ((lane & 3) == 0) red[threadIdx.x >> 6][lane >> 2] = s;
-  __syncthreads();
-  s = 0.0;
-  if (threadIdx.x < 16)
-#pragma unroll
-    for (int i = 0; i < NW; ++i) s += red[i][threadIdx.x];
-  return s;
-}
-
 // 1 / D per fine cell and their sum; starts the flag of the cell.
 template <int M>
 __global__ __launch_bounds__(1024) void nrt_seq_weights_kernel(NrtSeq g) {
@@ -206,7 +172,7 @@ __global__ __launch_bounds__(1024) void nrt_seq_weights_kernel(NrtSeq g) {
     W[c] = w;
     sum += w;
   }
-  sum = wsum(sum);
+  sum = wave_sum(sum);
   bad = __any(bad);
   if ((tid & 63) == 0) {
     red[tid >> 6] = sum;
@@ -597,6 +563,8 @@ hipError_t launch(int l, const NrtSeq& g, hipStream_t s, hipEvent_t* mid) {
   rw.rhs = g.rhs;
   rw.bad = g.general;
   rw.n_cells = g.n_cells;
+  rw.nr = 12;
+  rw.edge = true;
   SEQ_HIP(msfec_detail::q1t_rows(l, rw, s));
   if (mid) SEQ_HIP(hipEventRecord(mid[0], s));
   msfec_detail::Q1tCg cg{};
@@ -607,6 +575,7 @@ hipError_t launch(int l, const NrtSeq& g, hipStream_t s, hipEvent_t* mid) {
   cg.iters = g.iters;
   cg.n_cells = g.n_cells;
   cg.nr = 12;
+  cg.direct = true;
   cg.max_iter = g.max_iter;
   cg.tol = g.rtol;
   SEQ_HIP(msfec_detail::q1t_solve(l, cg, s));

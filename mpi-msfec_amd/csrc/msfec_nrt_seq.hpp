@@ -11,7 +11,7 @@ struct NrtSeq {
   const double* bq;     // n_cells x M^3 x 8
   const double* fq;     // n_cells x M^3 x 8 x 3, or null
   double* W;            // n_cells x (M^3 + 1): 1 / (integral of B / |c|^2) per fine cell, and their sum
-  double* st;           // n_cells x 27 x M^3
+  double* st;           // n_cells x 15 x M^3
   double* rhs;          // n_cells x 12 x M^3
   double* phi;          // n_cells x 12 x M^3
   int* iters;           // n_cells x 12 x 2

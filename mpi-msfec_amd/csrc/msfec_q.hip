@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "msfec.h"
+#include "msfec_q1t.hpp"
 
 namespace {
 
@@ -4203,6 +4204,7 @@ struct msfec_q_batch {
   int* d_status = nullptr;
   int* d_inode = nullptr;
   unsigned* d_imask = nullptr;
+  double* d_q1t = nullptr;  // 3-D CG on assembled rows: rows, right-hand sides, values, partial sums, ints
   size_t bytes = 0;
   bool coef_set = false, rhs_set = false, reac_set = false, computed = false;
   hipStream_t stream = nullptr;
@@ -4235,7 +4237,7 @@ void free_all(msfec_q_batch* h) {
   void* ptrs[] = {h->d_pb,    h->d_conv,  h->d_cgit,  h->d_rres,  h->d_rows,  h->d_verts, h->d_coef, h->d_f,     h->d_reac,  h->d_slo,   h->d_F,
                   h->d_rhs,   h->d_L,    h->d_W,     h->d_X,     h->d_psi,   h->d_M,
                   h->d_b,     h->d_status, h->d_inode, h->d_imask, h->d_cK,  h->d_crhs,
-                  h->d_cvec,  h->d_cit};
+                  h->d_cvec,  h->d_cit,  h->d_q1t};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (auto& set : h->ev_sets)
@@ -4513,11 +4515,17 @@ msfec_status msfec_q_create(const msfec_q_params* params, int n_cells, const dou
     TRY(dalloc(h, &h->d_rres, (size_t)n_cells * c.n * kMaxNb));
     TRY(dalloc(h, &h->d_conv, (size_t)n_cells));
   }
+  // tensors or Gauss-point loads under CG in 3-D: rows and solution of msfec_q1t.hip
+  const bool q1t = p.solver == MSFEC_SOLVER_CG && !h->fast && p.dim == 3;
   if (p.solver == MSFEC_SOLVER_CG) {
-    TRY(dalloc(h, &h->d_rres, (size_t)n_cells * c.n * kMaxNb));
+    if (!q1t) TRY(dalloc(h, &h->d_rres, (size_t)n_cells * c.n * kMaxNb));
     TRY(dalloc(h, &h->d_cgit, (size_t)n_cells * nv * 2));
   }
-  if (!h->fast) {
+  if (q1t) {
+    const size_t slabs = (size_t)msfec_detail::q1t_slabs(p.n_refine_local);
+    TRY(dalloc(h, &h->d_q1t, (size_t)n_cells * ((size_t)c.nfc * (15 + 8 + 8) + slabs * 48 + 8)));
+  }
+  if (!h->fast && !q1t) {
     TRY(dalloc(h, &h->d_slo, (size_t)n_cells * c.nn * c.nlow));
     TRY(dalloc(h, &h->d_F, (size_t)n_cells * c.nn));
     TRY(dalloc(h, &h->d_rhs, (size_t)n_cells * c.n * kMaxNb));
@@ -4529,7 +4537,7 @@ msfec_status msfec_q_create(const msfec_q_params* params, int n_cells, const dou
     TRY(dalloc(h, &h->d_L, (size_t)n_cells * std::max((size_t)c.n * kWin, nq * 256)));
     TRY(dalloc(h, &h->d_W, (size_t)n_cells * std::max((size_t)c.n * kMaxNb, nq * 32)));
   }
-  TRY(dalloc(h, &h->d_X, (size_t)n_cells * c.n * kMaxNb));
+  if (!q1t) TRY(dalloc(h, &h->d_X, (size_t)n_cells * c.n * kMaxNb));
   TRY(dalloc(h, &h->d_psi, (size_t)n_cells * nv * c.nn));
   TRY(dalloc(h, &h->d_M, (size_t)n_cells * nv * nv));
   TRY(dalloc(h, &h->d_b, (size_t)n_cells * nv));
@@ -4672,6 +4680,58 @@ msfec_status msfec_q_compute(msfec_q_handle h, void* stream) {
 #undef LAUNCH_ROWS
     MSFEC_HIP(hipGetLastError());
   }
+  if (h->d_q1t) {
+    msfec_detail::Q1tRows rw{};
+    const size_t nz = (size_t)h->n_cells * c.nfc;
+    rw.verts = h->d_verts;
+    rw.a = h->d_coef;
+    rw.reac = h->reac_count ? h->d_reac : nullptr;
+    rw.st = h->d_q1t;
+    rw.rhs = rw.st + 15 * nz;
+    rw.n_cells = h->n_cells;
+    rw.nr = c.reaction_mode == MSFEC_REACTION_NONE ? 7 : 8;
+    rw.scalar = c.coef_mode == MSFEC_COEF_SCALAR_CELL;
+    rw.reac0 = c.reaction_mode == MSFEC_REACTION_CONST ? c.reaction_const : 0.0;
+    MSFEC_HIP(msfec_detail::q1t_rows(h->p.n_refine_local, rw, s));
+    if (tm) MSFEC_HIP(hipEventRecord(ev[1], s));
+    msfec_detail::Q1tCg cg{};
+    cg.st = rw.st;
+    cg.rhs = rw.rhs;
+    cg.x = rw.rhs + 8 * nz;
+    double* part = cg.x + 8 * nz;
+    cg.iters = reinterpret_cast<int*>(
+        part + (size_t)h->n_cells * msfec_detail::q1t_slabs(h->p.n_refine_local) * 48);
+    cg.n_cells = h->n_cells;
+    cg.nr = rw.nr;
+    cg.max_iter = h->p.cg_max_iter > 0 ? h->p.cg_max_iter : 5000;
+    cg.tol = h->p.cg_tol > 0.0 ? h->p.cg_tol : 1e-13;
+    MSFEC_HIP(msfec_detail::q1t_solve(h->p.n_refine_local, cg, s));
+    if (tm) MSFEC_HIP(hipEventRecord(ev[2], s));
+    msfec_detail::Q1tBasis bs{};
+    bs.verts = rw.verts;
+    bs.a = rw.a;
+    bs.reac = rw.reac;
+    bs.f = h->rhs_count ? h->d_f : nullptr;
+    bs.x = cg.x;
+    bs.iters = cg.iters;
+    bs.part = part;
+    bs.Psi = h->d_psi;
+    bs.Mat = h->d_M;
+    bs.b = h->d_b;
+    bs.cgit = h->d_cgit;
+    bs.status = h->d_status;
+    bs.n_cells = h->n_cells;
+    bs.nr = cg.nr;
+    bs.per_point = c.rhs_mode == MSFEC_RHS_QP ? 8 : 1;
+    bs.scalar = rw.scalar;
+    bs.reac0 = rw.reac0;
+    bs.f0 = c.rhs_const;
+    MSFEC_HIP(msfec_detail::q1t_basis(h->p.n_refine_local, bs, s));
+    if (tm)
+      for (int i = 3; i < 6; ++i) MSFEC_HIP(hipEventRecord(ev[i], s));
+    h->computed = true;
+    return MSFEC_OK;
+  }
   if (!fast) {
     hipLaunchKernelGGL(q_assemble_kernel, dim3(h->n_cells), dim3(256), 0, s, c, h->d_verts,
                        h->d_coef, cstride, h->rhs_count ? h->d_f : nullptr, fstride,
@@ -4688,7 +4748,7 @@ msfec_status msfec_q_compute(msfec_q_handle h, void* stream) {
                           : 0;
 #define LAUNCH_BAND(K, D, F) hipLaunchKernelGGL((K<D, F>), dim3(h->n_cells), dim3(64), dyn, s, a)
   if (h->p.solver == MSFEC_SOLVER_CG && !fast) {
-    // tensor coefficients / Gauss-point loads: CG on the assembled stencil
+    // tensor coefficients / Gauss-point loads in 2-D: CG on the assembled stencil
     CgArgs g{};
     g.tol = h->p.cg_tol > 0.0 ? h->p.cg_tol : 1e-13;
     g.max_iter = h->p.cg_max_iter > 0 ? h->p.cg_max_iter : 5000;
@@ -4705,23 +4765,16 @@ msfec_status msfec_q_compute(msfec_q_handle h, void* stream) {
     hipLaunchKernelGGL((q_cg_stencil_kernel<D>), dim3(h->n_cells * g.nsolve), dim3(kCgThreads), \
                        cdyn, s, a, g, c);                                                 \
   } while (0)
-    if (c.dim == 3) LAUNCH_CGS(3);
-    else LAUNCH_CGS(2);
+    LAUNCH_CGS(2);
 #undef LAUNCH_CGS
     MSFEC_HIP(hipGetLastError());
     if (!reac) {
       const unsigned ub = (unsigned)(((size_t)h->n_cells * c.n + 255) / 256);
-      if (c.dim == 3)
-        hipLaunchKernelGGL((q_cg_unity_kernel<3>), dim3(ub), dim3(256), 0, s, a, g, h->n_cells);
-      else
-        hipLaunchKernelGGL((q_cg_unity_kernel<2>), dim3(ub), dim3(256), 0, s, a, g, h->n_cells);
+      hipLaunchKernelGGL((q_cg_unity_kernel<2>), dim3(ub), dim3(256), 0, s, a, g, h->n_cells);
       MSFEC_HIP(hipGetLastError());
     }
     if (tm) MSFEC_HIP(hipEventRecord(ev[2], s));
-    if (c.dim == 3)
-      hipLaunchKernelGGL((q_cg_tensor_finish_kernel<3>), dim3(h->n_cells), dim3(kTfThreads), 0, s, a, g, c);
-    else
-      hipLaunchKernelGGL((q_cg_tensor_finish_kernel<2>), dim3(h->n_cells), dim3(kTfThreads), 0, s, a, g, c);
+    hipLaunchKernelGGL((q_cg_tensor_finish_kernel<2>), dim3(h->n_cells), dim3(kTfThreads), 0, s, a, g, c);
     MSFEC_HIP(hipGetLastError());
     if (tm) MSFEC_HIP(hipEventRecord(ev[3], s));
   } else if (h->p.solver == MSFEC_SOLVER_CG) {
