@@ -597,15 +597,18 @@ msfec_status msfec_nrt_destroy(msfec_nrt_handle h);
  * Raviart-Thomas x DQ0 system per coarse box cell, on the 2^l x 2^l x 2^l
  * fine grid (fine faces numbered as the faces of the Ned_RT section without
  * the edge offset: nf = 3 m^2 (m+1)).  The flux of basis n is the coarse
- * Raviart-Thomas function of face n plus the curl of an interior Nedelec
- * field, solved by Jacobi-PCG on the curl-curl system; u is 1
- * (set_u_to_std).  No reaction term (the reference's ReactionRate is zero).
+ * Raviart-Thomas function of face n plus a divergence-free flux, solved by
+ * conjugate gradients on those fluxes (preconditioned by the projection in
+ * the plain face mass) or, for a cell whose A^-1 has a very high contrast or
+ * is not positive definite, on the curl-curl system of a potential
+ * (Jacobi); u is 1 (set_u_to_std).  No reaction term (the reference's ReactionRate is zero).
  * ------------------------------------------------------------------------- */
 typedef struct {
   int n_refine_local; /* l, 1..4                                                  */
   int flags;          /* MSFEC_FLAG_*                                             */
   int max_iter;       /* CG iteration limit, 0: 20000 (MSFEC_CELL_NOT_CONVERGED) */
-  double rtol;        /* CG stop: |r| <= rtol |b|, 0: 1e-13                       */
+  double rtol;        /* CG stop: preconditioned residual (curl-curl: residual) <=
+                         rtol x the initial one, 0: 1e-13                        */
 } msfec_rt3_params;
 
 typedef struct msfec_rt3_batch *msfec_rt3_handle;

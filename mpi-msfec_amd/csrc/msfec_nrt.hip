@@ -55,6 +55,7 @@
 
 #include "msfec.h"
 #include "msfec_nrt_seq.hpp"
+#include "msfec_rt3_proj.hpp"
 
 namespace msfec_detail {
 extern thread_local std::string g_last_error;
@@ -1916,7 +1917,7 @@ struct Rt3Args {
   const double* verts;  // n_cells x 8 x 3
   const double* ainv;   // n_cells x nfc x 8 x 6
   const double* fq;     // n_cells x nfc x 8, or null
-  double* MF;           // n_cells x 21 x nfc: face mass with A^-1 per fine cell (colour-major)
+  double* MF;           // n_cells x 22 x nfc (the last unused): face mass with A^-1 per fine cell (colour-major)
   double* PD;           // n_cells x ns: inverse Jacobi diagonal
   double* WK;           // n_cells x 6 x 4 x ns: x, r, p, q over the interior edges
   double* S;            // n_cells x 6 x nf: the fine fluxes
@@ -1924,7 +1925,7 @@ struct Rt3Args {
   double* b;            // n_cells x 7
   int* its;             // n_cells x 6
   int* flg;             // n_cells x 6
-  int* status;          // n_cells
+  const int* need;      // n_cells: the cells computed here
   int n_cells, ns, max_iter;
   double rtol;
 };
@@ -1986,10 +1987,11 @@ template <int L>
 __global__ __launch_bounds__(256) void rt3_local_kernel(Rt3Args g) {
   constexpr int M = 1 << L, nfc = M * M * M;
   const int cell = blockIdx.x;
+  if (!g.need[cell]) return;
   V3 Hc, h;
   it_sizes(g.verts + (size_t)cell * 24, Hc, h, M);
   const double w8 = h.x * h.y * h.z * 0.125;
-  double* mf = g.MF + (size_t)cell * 21 * nfc;
+  double* mf = g.MF + (size_t)cell * 22 * nfc;
   for (int idx = threadIdx.x; idx < nfc * 21; idx += 256) {
     const int e = idx / nfc, c = idx - e * nfc;
     int F, G;
@@ -2011,7 +2013,8 @@ template <int L>
 __global__ __launch_bounds__(256) void rt3_diag_kernel(Rt3Args g) {
   constexpr int M = 1 << L, nfc = M * M * M, ne = 3 * M * (M + 1) * (M + 1);
   const int cell = blockIdx.x;
-  const double* mf = g.MF + (size_t)cell * 21 * nfc;
+  if (!g.need[cell]) return;
+  const double* mf = g.MF + (size_t)cell * 22 * nfc;
   double* pd = g.PD + (size_t)cell * g.ns;
   for (int e = threadIdx.x; e < ne; e += 256) {
     int t, p0, p1, p2;
@@ -2106,9 +2109,9 @@ __global__ __launch_bounds__(kItNT) void rt3_cg_kernel(Rt3Args g) {
   __shared__ double redA[kItNW], redB[2 * kItNW];
   const int bid = blockIdx.x, slot = bid >> 3;
   const int cell = (slot / 6) * 8 + (bid & 7), nb = slot % 6;
-  if (cell >= g.n_cells) return;
+  if (cell >= g.n_cells || !g.need[cell]) return;
   const int tid = threadIdx.x;
-  const double* mf = g.MF + (size_t)cell * 21 * nfc;
+  const double* mf = g.MF + (size_t)cell * 22 * nfc;
   const double* pd = g.PD + (size_t)cell * ns;
   double* x = g.WK + ((size_t)cell * 6 + nb) * 4 * ns;
   double* r = x + ns;
@@ -2238,7 +2241,8 @@ __global__ __launch_bounds__(256) void rt3_element_kernel(Rt3Args g) {
   constexpr int M = 1 << L, nfc = M * M * M, nf = 3 * M * M * (M + 1);
   __shared__ double red[4][8];
   const int cell = blockIdx.x / 7, i = blockIdx.x % 7, tid = threadIdx.x;
-  const double* mf = g.MF + (size_t)cell * 21 * nfc;
+  if (!g.need[cell]) return;
+  const double* mf = g.MF + (size_t)cell * 22 * nfc;
   const double* S = g.S + (size_t)cell * 6 * nf;
   double acc[8];
 #pragma unroll
@@ -2307,19 +2311,6 @@ __global__ __launch_bounds__(256) void rt3_element_kernel(Rt3Args g) {
       bc[6] = t[7];
     }
   }
-}
-
-__global__ __launch_bounds__(256) void rt3_status_kernel(Rt3Args g) {
-  const int cell = blockIdx.x * 256 + threadIdx.x;
-  if (cell >= g.n_cells) return;
-  int st = MSFEC_CELL_OK;
-  for (int n = 0; n < 6; ++n) {
-    const int f = g.flg[(size_t)cell * 6 + n];
-    if (f != MSFEC_CELL_OK && st == MSFEC_CELL_OK) st = f;
-  }
-  for (int k = 0; k < 49 && st == MSFEC_CELL_OK; ++k)
-    if (!isfinite(g.M[(size_t)cell * 49 + k])) st = MSFEC_CELL_NONFINITE;
-  g.status[cell] = st;
 }
 
 msfec_status nrt_fail(msfec_status st, const std::string& msg) {
@@ -2978,6 +2969,8 @@ struct msfec_rt3_batch {
   double* d_ainv = nullptr;
   double* d_f = nullptr;
   double* d_MF = nullptr;
+  double* d_proj = nullptr;  // bounds and partial sums
+  int* d_gen = nullptr;
   double* d_PD = nullptr;
   double* d_WK = nullptr;
   double* d_S = nullptr;
@@ -2996,7 +2989,8 @@ namespace {
 
 void rt3_free(msfec_rt3_batch* h) {
   void* ptrs[] = {h->d_verts, h->d_ainv, h->d_f,   h->d_MF,  h->d_PD,    h->d_WK,
-                  h->d_S,     h->d_M,    h->d_b,   h->d_its, h->d_flg, h->d_status};
+                  h->d_S,     h->d_M,    h->d_b,   h->d_its, h->d_flg, h->d_status,
+                  h->d_proj, h->d_gen};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (auto& set : h->ev_sets)
@@ -3019,25 +3013,45 @@ msfec_status rt3_launch(msfec_rt3_batch* h, hipStream_t s, std::array<hipEvent_t
   a.b = h->d_b;
   a.its = h->d_its;
   a.flg = h->d_flg;
-  a.status = h->d_status;
+  a.need = h->d_gen;
   a.n_cells = h->n_cells;
   a.ns = h->ns;
   a.max_iter = h->prm.max_iter > 0 ? h->prm.max_iter : 20000;
   a.rtol = h->prm.rtol > 0.0 ? h->prm.rtol : 1e-13;
   const int nc = h->n_cells;
+  msfec_detail::Rt3Proj q{};
+  q.verts = a.verts;
+  q.ainv = a.ainv;
+  q.fq = a.fq;
+  q.MF = h->d_MF;
+  q.bound = h->d_proj;
+  q.part = h->d_proj + (size_t)nc * msfec_detail::rt3_proj_blocks(L) * 2;
+  q.general = h->d_gen;
+  q.S = a.S;
+  q.Mat = a.M;
+  q.b = a.b;
+  q.its = a.its;
+  q.flg = a.flg;
+  q.status = h->d_status;
+  q.n_cells = nc;
+  q.max_iter = a.max_iter;
+  q.rtol = a.rtol;
+  NRT_HIP(msfec_detail::rt3_proj_masses(L, q, s));
+  if (ev) NRT_HIP(hipEventRecord((*ev)[1], s));
+  NRT_HIP(msfec_detail::rt3_proj_solve(L, q, s));
+  // the cells left over, on the curl-curl system; their workgroups leave the
+  // others at once
   hipLaunchKernelGGL(rt3_local_kernel<L>, dim3(nc), dim3(256), 0, s, a);
   NRT_HIP(hipGetLastError());
   hipLaunchKernelGGL(rt3_diag_kernel<L>, dim3(nc), dim3(256), 0, s, a);
   NRT_HIP(hipGetLastError());
-  if (ev) NRT_HIP(hipEventRecord((*ev)[1], s));
   const int groups = (nc + 7) / 8;
   hipLaunchKernelGGL(rt3_cg_kernel<L>, dim3(groups * 8 * 6), dim3(kItNT), 0, s, a);
   NRT_HIP(hipGetLastError());
   if (ev) NRT_HIP(hipEventRecord((*ev)[2], s));
   hipLaunchKernelGGL(rt3_element_kernel<L>, dim3(nc * 7), dim3(256), 0, s, a);
   NRT_HIP(hipGetLastError());
-  hipLaunchKernelGGL(rt3_status_kernel, dim3((nc + 255) / 256), dim3(256), 0, s, a);
-  NRT_HIP(hipGetLastError());
+  NRT_HIP(msfec_detail::rt3_proj_element(L, q, s));
   return MSFEC_OK;
 }
 
@@ -3099,7 +3113,9 @@ msfec_status msfec_rt3_create(const msfec_rt3_params* params, int n_cells, const
   RT3_TRY(nrt_alloc(&h->d_verts, nc * 24));
   RT3_TRY(nrt_alloc(&h->d_ainv, nc * nfc * 8 * 6));
   RT3_TRY(nrt_alloc(&h->d_f, nc * nfc * 8));
-  RT3_TRY(nrt_alloc(&h->d_MF, nc * 21 * nfc));
+  RT3_TRY(nrt_alloc(&h->d_MF, nc * 22 * nfc));
+  RT3_TRY(nrt_alloc(&h->d_proj, nc * msfec_detail::rt3_proj_blocks(l) * 34));
+  RT3_TRY(nrt_alloc(&h->d_gen, nc));
   RT3_TRY(nrt_alloc(&h->d_PD, nc * h->ns));
   RT3_TRY(nrt_alloc(&h->d_WK, nc * 6 * 4 * h->ns));
   RT3_TRY(nrt_alloc(&h->d_S, nc * 6 * h->nf));

@@ -34,11 +34,13 @@
 
 #include "msfec.h"
 #include "msfec_q1t.hpp"
+#include "msfec_trig.hpp"
 #include "msfec_wave.hpp"
 
 namespace {
 
 using msfec_detail::NrtSeq;
+using namespace msfec_trig;
 using msfec_wave::block_sums;
 using msfec_wave::wave_sum;
 
@@ -46,97 +48,6 @@ constexpr double kGp[2] = {0.21132486540518711775, 0.78867513459481288225};
 constexpr int kLnAx[12] = {1, 1, 0, 0, 1, 1, 0, 0, 2, 2, 2, 2};
 constexpr int kLnF1[12] = {0, 1, 0, 1, 0, 1, 0, 1, 0, 1, 0, 1};
 constexpr int kLnF2[12] = {0, 0, 0, 0, 1, 1, 1, 1, 0, 0, 1, 1};
-
-// cos(t pi / 32)
-__host__ __device__ constexpr double cos32(int t) {
-  t = ((t % 64) + 64) % 64;
-  if (t > 32) t = 64 - t;
-  const int u = t > 16 ? 32 - t : t;
-  const double c = u == 0    ? 1.0
-                   : u == 1  ? 0.99518472667219692873
-                   : u == 2  ? 0.98078528040323043058
-                   : u == 3  ? 0.95694033573220882438
-                   : u == 4  ? 0.92387953251128673848
-                   : u == 5  ? 0.88192126434835504956
-                   : u == 6  ? 0.83146961230254523567
-                   : u == 7  ? 0.77301045336273699338
-                   : u == 8  ? 0.70710678118654757274
-                   : u == 9  ? 0.63439328416364548779
-                   : u == 10 ? 0.55557023301960228867
-                   : u == 11 ? 0.47139673682599780857
-                   : u == 12 ? 0.38268343236508983729
-                   : u == 13 ? 0.29028467725446233105
-                   : u == 14 ? 0.19509032201612833135
-                   : u == 15 ? 0.098017140329560770162
-                             : 0.0;
-  return t > 16 ? -c : c;
-}
-// cos(t pi / 2M)
-template <int M>
-__host__ __device__ constexpr double cosm(int t) {
-  return cos32(t * (16 / M));
-}
-
-// One line of M values, in place; the even and the odd modes use the sums
-// and the differences of mirrored points, half the products of the full
-// matrix.
-//   sine: points and modes 1 .. M-1 (index 0 is not read, and zero after)
-template <int M>
-__device__ __forceinline__ void sine_line(double* v) {
-  constexpr int H = M / 2;
-  double s[H], d[H];
-#pragma unroll
-  for (int j = 1; j < H; ++j) {
-    s[j] = v[j] + v[M - j];
-    d[j] = v[j] - v[M - j];
-  }
-  const double mid = v[H];
-  v[0] = 0.0;
-#pragma unroll
-  for (int k = 1; k < M; ++k) {
-    double a = k & 1 ? mid * cosm<M>(M - 2 * H * k) : 0.0;
-#pragma unroll
-    for (int j = 1; j < H; ++j) a = fma(cosm<M>(M - 2 * j * k), k & 1 ? s[j] : d[j], a);
-    v[k] = a;
-  }
-}
-//   cosine: M cell values to modes 0 .. M-1
-template <int M>
-__device__ __forceinline__ void cos_line(double* v) {
-  constexpr int H = M / 2;
-  double s[H], d[H];
-#pragma unroll
-  for (int c = 0; c < H; ++c) {
-    s[c] = v[c] + v[M - 1 - c];
-    d[c] = v[c] - v[M - 1 - c];
-  }
-#pragma unroll
-  for (int k = 0; k < M; ++k) {
-    double a = 0.0;
-#pragma unroll
-    for (int c = 0; c < H; ++c) a = fma(cosm<M>((2 * c + 1) * k), k & 1 ? d[c] : s[c], a);
-    v[k] = a;
-  }
-}
-//   and back
-template <int M>
-__device__ __forceinline__ void cos_line_t(double* v) {
-  constexpr int H = M / 2;
-  double e[H], o[H];
-#pragma unroll
-  for (int c = 0; c < H; ++c) {
-    e[c] = o[c] = 0.0;
-#pragma unroll
-    for (int k = 0; k < M; k += 2) e[c] = fma(cosm<M>((2 * c + 1) * k), v[k], e[c]);
-#pragma unroll
-    for (int k = 1; k < M; k += 2) o[c] = fma(cosm<M>((2 * c + 1) * k), v[k], o[c]);
-  }
-#pragma unroll
-  for (int c = 0; c < H; ++c) {
-    v[c] = e[c] + o[c];
-    v[M - 1 - c] = e[c] - o[c];
-  }
-}
 
 template <int M>
 struct Seq {
@@ -209,37 +120,6 @@ __device__ __forceinline__ int edge_at(int a, int i, int j, int k) {
   if (a == 0) return (k * S + j) * M + i;
   if (a == 1) return NX + (k * M + j) * S + i;
   return 2 * NX + (k * S + j) * S + i;
-}
-
-// the three transforms of one component (axis a) in both directions: an
-// edge field is a cosine along its axis and a sine across it, a face field
-// the other way round
-template <int M, bool Forward>
-__device__ __forceinline__ void transform(double* E, int comps) {
-  constexpr int S = M + 1, S3 = S * S * S, M2 = M * M, NT = Seq<M>::NT;
-#pragma unroll 1
-  for (int d = 0; d < 3; ++d) {
-    const int step = d == 0 ? 1 : (d == 1 ? S : S * S);
-    for (int ln = threadIdx.x; ln < comps * M2; ln += NT) {
-      const int a = ln / M2, u = ln % M, w = (ln / M) % M;
-      // lines along x: neighbouring lanes S values apart (no bank conflict,
-      // S is odd); along y and z: neighbouring values
-      double* p = E + a * S3 + (d == 0 ? (w * S + u) * S : (d == 1 ? w * S * S + u : w * S + u));
-      double v[M];
-#pragma unroll
-      for (int t = 0; t < M; ++t) v[t] = p[t * step];
-      if constexpr (Forward) {
-        if (a == d || comps == 1) cos_line<M>(v);
-        else sine_line<M>(v);
-      } else {
-        if (a == d) sine_line<M>(v);
-        else cos_line_t<M>(v);
-      }
-#pragma unroll
-      for (int t = 0; t < M; ++t) p[t * step] = v[t];
-    }
-    __syncthreads();
-  }
 }
 
 // Workgroup n of a coarse cell: n < 12 the edge basis n, with its column of
@@ -384,7 +264,7 @@ __global__ __launch_bounds__(Seq<M>::NT) void nrt_seq_basis_kernel(NrtSeq g) {
     }
     const double col = block_sums<Q::NW>(acc, red);
     if (tid < 12) Mc[tid * 18 + n] = col;
-    transform<M, true>(E, 3);
+    transform<M, NT, EdgeToModes>(E, 3);
   } else {
     // d' = 1/D over its sum - 1/M^3: the divergence of the +1 faces less
     // that of the coarse function
@@ -393,7 +273,7 @@ __global__ __launch_bounds__(Seq<M>::NT) void nrt_seq_basis_kernel(NrtSeq g) {
     for (int c = tid; c < M3; c += NT)
       E[((c / (M * M)) * S + (c / M) % M) * S + c % M] = fma(W[c], sc, -1.0 / M3);
     __syncthreads();
-    transform<M, true>(E, 1);
+    transform<M, NT, CellToModes>(E, 1);
   }
   for (int c = tid; c < M3; c += NT) {
     const int kx = c % M, ky = (c / M) % M, kz = c / (M * M);
@@ -426,7 +306,7 @@ __global__ __launch_bounds__(Seq<M>::NT) void nrt_seq_basis_kernel(NrtSeq g) {
     p[2 * S3] = u[2];
   }
   __syncthreads();
-  transform<M, false>(E, 3);
+  transform<M, NT, ModesToFace>(E, 3);
   // the faces of the basis (or of the 6 face bases, c_n +- u*)
   double acc[16];
 #pragma unroll

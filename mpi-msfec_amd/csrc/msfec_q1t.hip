@@ -13,6 +13,8 @@ using msfec_detail::Q1tBasis;
 using msfec_detail::Q1tCg;
 using msfec_detail::Q1tRows;
 using msfec_wave::block_sums;
+using msfec_wave::from_left;
+using msfec_wave::from_right;
 using msfec_wave::wave_sum;
 
 constexpr double kGp[2] = {0.21132486540518711775, 0.78867513459481288225};
@@ -183,18 +185,6 @@ typedef unsigned row_v2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ double row_entry(__amdgpu_buffer_rsrc_t rsrc, int lane, int uni) {
   const row_v2 t = __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane, uni, 0);
   return __hiloint2double((int)t.y, (int)t.x);
-}
-
-// v of the lane to the right (left); zero at the ends of a row of 16 lanes
-__device__ __forceinline__ double from_right(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x101, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x101, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double from_left(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x111, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x111, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
 }
 
 // Jacobi-preconditioned conjugate gradients, one right-hand side of one

@@ -1,4 +1,4 @@
-// Sums over a wave and a workgroup.
+// Lane shifts, and sums over a wave and a workgroup.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -8,6 +8,18 @@ __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
   return v;
+}
+
+// v of the lane to the right (left); zero at the ends of a row of 16 lanes
+__device__ __forceinline__ double from_right(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x101, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x101, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double from_left(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x111, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x111, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
 }
 
 // Block sums of 16 values per thread; thread t < 16 returns the t-th (red is

@@ -1,0 +1,71 @@
+"""The 3-D RT_DQ fluxes by projected conjugate gradients, on every grid size of
+the kernels and on both sides of the contrast above which the curl-curl solver
+takes a cell."""
+import numpy as np
+import pytest
+
+from test_gpu_nrt import boxes, rand_coefs
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.abs(a - b).max() / np.abs(b).max()
+
+
+def run(verts, l, ainv, f=None, **kw):
+    from msfec_amd import RTDQ3BasisBatch
+    with RTDQ3BasisBatch(verts, n_refine_local=l, **kw) as rb:
+        rb.set_coefficients(ainv, f)
+        rb.run()
+        return (rb.get_global_element_matrix(), rb.get_global_element_rhs(), rb.get_basis(),
+                rb.get_cell_status(), rb.get_iterations())
+
+
+@pytest.mark.parametrize("l,n", [(1, 17), (2, 9), (3, 3)])
+def test_contrasts_in_one_batch(oracle_mod, l, n):
+    """Stretched boxes with rotated tensors, cell c scaled by lognormal factors
+    of deviation 0, 1, 2, .. 6 in turn (contrast 1e1 to beyond 1e8: the last
+    ones are left to the curl-curl solver).  1e-9 on fluxes and matrix, the
+    tolerance of the other 3-D RT_DQ tests; for the two largest contrasts
+    1e-7: there both methods stop at 1e-13 of a residual that the contrast
+    amplifies."""
+    print(f"case rt3 contrasts l={l} n={n}", flush=True)
+    rng = np.random.default_rng(5000 + l)
+    verts = boxes(rng, n)
+    ainv, _, _, _ = rand_coefs(rng, n, l, reaction=False, load=False)
+    f = rng.normal(size=(n, 8 ** l, 8))
+    dev = np.arange(n) % 7
+    ainv = ainv * np.exp(dev[:, None, None, None] * rng.normal(size=ainv.shape[:2] + (1, 1)))
+    M, b, S, st, its = run(verts, l, ainv, f)
+    assert (st == 0).all(), st
+    for c in range(n):
+        Mo, bo, So, sto = oracle_mod.rt3_basis_cell(l, verts[c], ainv[c], f[c])
+        assert sto == 0
+        tol = 1e-9 if dev[c] < 5 else 1e-7
+        es = max(rel(S[c, i], So[i]) for i in range(6))
+        print(f"cell {c} deviation {dev[c]}: {es:.1e} {rel(M[c], Mo):.1e} its {its[c].max()}", flush=True)
+        assert es <= tol and rel(M[c], Mo) <= tol and rel(b[c], bo) <= 1e-12
+
+
+@pytest.mark.parametrize("l", [2, 3, 4])
+def test_general_cells_do_not_disturb_others(l):
+    """Cells that go to the curl-curl solver (indefinite, NaN, huge contrast)
+    between cells that do not: the latter come out bit for bit as without
+    them."""
+    print(f"case rt3 neighbours of general cells l={l}", flush=True)
+    rng = np.random.default_rng(5100 + l)
+    n = 10
+    verts = boxes(rng, n)
+    ainv, _, _, _ = rand_coefs(rng, n, l, reaction=False, load=False)
+    good = run(verts, l, ainv, max_iter=300)
+    ainv[1] = -ainv[1]
+    ainv[4, 3, 2, 0] = np.nan
+    ainv[7, ::2] *= 1e9
+    ainv[9, 0, 0, 3] = -1e-3
+    got = run(verts, l, ainv, max_iter=300)
+    assert got[3][1] != 0 and got[3][4] != 0
+    for c in (0, 2, 3, 5, 6, 8):
+        assert got[3][c] == 0
+        for k in range(3):
+            np.testing.assert_array_equal(got[k][c], good[k][c])
