@@ -25,7 +25,7 @@
 // edges and faces.  Measured, a whole pass with its copies: 4096 cells at l = 2
 // 6.81 ms by the dense factorisation, 0.73 ms here; 8 cells at l = 4 with the
 // contrast 0.9 of the reference example 345 ms by MINRES (773 iterations),
-// 1.37 ms here (50 iterations of CG).
+// 0.95 ms here (50 iterations of CG).
 //
 // That needs A^-1 positive definite at every Gauss point and B > 0 (and
 // finite data): a cell that is not so is flagged and left to the general

@@ -35,6 +35,7 @@
 
 #include "msfec.h"
 #include "msfec_q1t.hpp"
+#include "msfec_wave.hpp"
 
 namespace {
 
@@ -3274,6 +3275,8 @@ __global__ void coarse_weights_kernel(int dim, int nc, const double* __restrict_
 constexpr int kCgThreads = 512;
 constexpr int kCgOwn = 8;
 constexpr int kCgWaves = kCgThreads / 64;
+using msfec_wave::wave_sum;
+using msfec_wave::waves_sum;
 
 struct CgArgs {
   double tol;
@@ -3285,36 +3288,25 @@ struct CgArgs {
   const double* fnode;  // assembled-stencil path: nodal load [cells][nn]
 };
 
-// sum over the 64 lanes of the wave: DPP inside rows of 16, then across rows
-__device__ __forceinline__ double cg_wave_sum(double v) {
-  v += dpp_f64(v, 0);
-  v += dpp_f64(v, 1);
-  v += dpp_f64(v, 2);
-  v += __shfl_xor(v, 8);
-  v += __shfl_xor(v, 16);
-  v += __shfl_xor(v, 32);
-  return v;
-}
-
 // block sums of two values; every thread gets both.  One barrier: a caller
 // reuses a buffer only after a later barrier (two buffers in turn).
-__device__ __forceinline__ void cg_block_sum2(double& x, double& y, double (*red)[2]) {
-  x = cg_wave_sum(x);
-  y = cg_wave_sum(y);
+__device__ __forceinline__ void cg_block_sum2(double& x, double& y, double (*red)[kCgWaves]) {
+  x = wave_sum(x);
+  y = wave_sum(y);
   const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
-    red[w][0] = x;
-    red[w][1] = y;
+    red[0][w] = x;
+    red[1][w] = y;
   }
   __syncthreads();
-  double sx = 0.0, sy = 0.0;
-#pragma unroll
-  for (int i = 0; i < kCgWaves; ++i) {
-    sx += red[i][0];
-    sy += red[i][1];
-  }
-  x = sx;
-  y = sy;
+  x = waves_sum<kCgWaves>(red[0]);
+  y = waves_sum<kCgWaves>(red[1]);
+}
+__device__ __forceinline__ double cg_block_sum(double x, double* red) {
+  x = wave_sum(x);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  return waves_sum<kCgWaves>(red);
 }
 
 // K v at the rows of one segment (nodes (x0 .. x0 + len - 1, y, z), all
@@ -3469,7 +3461,7 @@ __global__ __launch_bounds__(kCgThreads) void q_cg_kernel(BandArgs a, CgArgs g) 
   // the two block sums of an iteration use one buffer each: the barrier of
   // the other sum (or the one closing the iteration) separates the reads of
   // a buffer from its next writes
-  __shared__ double red[2][kCgWaves][2];
+  __shared__ double red[2][2][kCgWaves];
   const bool has_rf = (a.reaction_mode == MSFEC_REACTION_CELL);
   double* cf = dyn;
   double* rf = dyn + a.nfc;
@@ -3567,11 +3559,11 @@ __global__ __launch_bounds__(kCgThreads) void q_cg_kernel(BandArgs a, CgArgs g) 
     }
     double q[kCgOwn];
     cg_line_apply<DIM, REAC>(cf, rf, has_rf, rc, kr, mr, x0, cy, cz, len, a.N, a.S, pv, q);
-    double pq = 0.0, dummy = 0.0;
+    double pq = 0.0;
 #pragma unroll
     for (int t = 0; t < kCgOwn; ++t)
       if (t < len) pq = fma(p[t], q[t], pq);
-    cg_block_sum2(pq, dummy, red[0]);
+    pq = cg_block_sum(pq, red[0][0]);
     if (!(pq > 0.0)) {
       state = 2;
       break;
@@ -3768,7 +3760,7 @@ __global__ __launch_bounds__(kCgThreads) void q_cg_stencil_kernel(BandArgs a, Cg
   const int cell = blockIdx.x / g.nsolve, j = blockIdx.x - cell * g.nsolve;
   const int tid = threadIdx.x;
   extern __shared__ double dyn[];  // search direction over all nodes
-  __shared__ double red[2][kCgWaves][2];
+  __shared__ double red[2][2][kCgWaves];
   __shared__ int off[D::NLOW];
   double* pv = dyn;
   if (tid < D::NLOW) off[tid] = c.off_full[tid];
@@ -3811,11 +3803,11 @@ __global__ __launch_bounds__(kCgThreads) void q_cg_stencil_kernel(BandArgs a, Cg
     double q[kCgOwn];
 #pragma unroll
     for (int t = 0; t < kCgOwn; ++t) q[t] = (t < len) ? cg_stencil_row<DIM>(slo, off, node0 + t, pv) : 0.0;
-    double pq = 0.0, dummy = 0.0;
+    double pq = 0.0;
 #pragma unroll
     for (int t = 0; t < kCgOwn; ++t)
       if (t < len) pq = fma(p[t], q[t], pq);
-    cg_block_sum2(pq, dummy, red[0]);
+    pq = cg_block_sum(pq, red[0][0]);
     if (!(pq > 0.0)) {
       state = 2;
       break;
@@ -3961,7 +3953,7 @@ __global__ __launch_bounds__(kTfThreads) void q_cg_tensor_finish_kernel(BandArgs
   const int w = tid >> 6, lane = tid & 63;
 #pragma unroll
   for (int t = 0; t < D::NV * D::NV + D::NV; ++t) {
-    const double v = cg_wave_sum(acc[t]);
+    const double v = wave_sum(acc[t]);
     if (lane == 0) part[w][t] = v;
   }
   __syncthreads();

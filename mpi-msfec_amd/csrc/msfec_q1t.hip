@@ -200,7 +200,7 @@ __device__ __forceinline__ double row_entry(__amdgpu_buffer_rsrc_t rsrc, int lan
 // workgroup at M = 16, 14.6 us), and 8 cells of rows an XCD then exceed its
 // L2 (64 cells x 7 bases: 2.4 ms with one vector per workgroup, 8.5 ms with
 // two sharing the rows, which keeps all 8 cells in use at once).  Here 9.7 us
-// an iteration: 1.54 ms for those, 0.75 ms for 8 cells x 12 potentials.
+// an iteration: 1.41 ms for those, 0.68 ms for 8 cells x 12 potentials.
 // Workgroups of one coarse cell share an XCD (block index mod 8).
 template <int M, int LZ>
 __global__ __launch_bounds__(M * M * M / LZ < 64 ? 64 : M * M * M / LZ) void q1t_cg_kernel(Q1tCg g) {

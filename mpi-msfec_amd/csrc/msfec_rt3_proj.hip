@@ -30,6 +30,7 @@ using msfec_wave::block_sums;
 using msfec_wave::from_left;
 using msfec_wave::from_right;
 using msfec_wave::wave_sum;
+using msfec_wave::waves_sum;
 using namespace msfec_trig;
 
 constexpr double kGp[2] = {0.21132486540518711775, 0.78867513459481288225};
@@ -297,10 +298,7 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
     if ((tid & 63) == 0) red[C::NW + (tid >> 6)] = rz;
     __syncthreads();
     transform<M, NT, ModesToFace>(E, 3);
-    rz = 0.0;
-#pragma unroll
-    for (int t = 0; t < C::NW; ++t) rz += red[C::NW + t];
-    return rz;
+    return waves_sum<C::NW>(red + C::NW);
   };
   apply(true);
   __syncthreads();
@@ -349,9 +347,7 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
     double pq = wave_sum(apply(false));
     if ((tid & 63) == 0) red[tid >> 6] = pq;
     __syncthreads();
-    pq = 0.0;
-#pragma unroll
-    for (int t = 0; t < C::NW; ++t) pq += red[t];
+    pq = waves_sum<C::NW>(red);
     if (!(pq > 0.0)) {
       flag = isfinite(pq) ? MSFEC_CELL_NOT_SPD : MSFEC_CELL_NONFINITE;
       break;

@@ -4,10 +4,40 @@
 
 namespace msfec_wave {
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+// Sum over the N lanes (a power of two, at most 16) of a row, or of N values
+// that repeat within it: every lane has it, in the same bits, as a + b = b + a.
+template <int N>
+__device__ __forceinline__ double row_sum(double v) {
+#define MSFEC_ROR(k)                                                                         \
+  if constexpr (N > k)                                                                       \
+    v += __hiloint2double(                                                                   \
+        __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + k, 0xf, 0xf, false),       \
+        __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + k, 0xf, 0xf, false))
+  MSFEC_ROR(8);
+  MSFEC_ROR(4);
+  MSFEC_ROR(2);
+  MSFEC_ROR(1);
+#undef MSFEC_ROR
   return v;
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// Sum over a wave, in every lane: by moves within the rows of 16 lanes and
+// scalar registers.  (The exchanges of __shfl_xor go through the LDS unit, six
+// round trips one after the other.  A pass of the CG kernels: 64 cells of 16^3
+// with tensors 1.71 ms with those, 1.58 ms so; 3-D RT_DQ, 64 cells, 3.79 and
+// 3.53 ms.)
+__device__ __forceinline__ double wave_sum(double v) {
+  v = row_sum<16>(v);
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+// Sum of the NW values at red (one of each wave), in every lane.
+template <int NW>
+__device__ __forceinline__ double waves_sum(const double* red) {
+  static_assert(NW <= 16, "one row");
+  return row_sum<NW>(red[threadIdx.x & (NW - 1)]);
 }
 
 // v of the lane to the right (left); zero at the ends of a row of 16 lanes
