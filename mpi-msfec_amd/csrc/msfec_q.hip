@@ -3083,28 +3083,20 @@ __global__ __launch_bounds__(1024) void coarse_cg_kernel(int dim, int nc, const 
   }
 }
 
-// Block sums of two values over the 16 waves of a 1024-thread workgroup;
-// every thread gets both.  One barrier: a caller reuses a buffer only after a
-// later barrier (two buffers in turn).
-__device__ __forceinline__ void coarse_block_sum2(double& x, double& y, double (*red)[2]) {
-  for (int o = 32; o > 0; o >>= 1) {
-    x += __shfl_xor(x, o);
-    y += __shfl_xor(y, o);
-  }
+// Block sums of two values over at most 16 waves (red holds zeros for those
+// that a smaller workgroup lacks); every thread gets both.  One barrier: a
+// caller reuses a buffer only after a later barrier (two buffers in turn).
+__device__ __forceinline__ void coarse_block_sum2(double& x, double& y, double (*red)[16]) {
+  x = msfec_wave::wave_sum(x);
+  y = msfec_wave::wave_sum(y);
   const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
-    red[w][0] = x;
-    red[w][1] = y;
+    red[0][w] = x;
+    red[1][w] = y;
   }
   __syncthreads();
-  double sx = 0.0, sy = 0.0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    sx += red[i][0];
-    sy += red[i][1];
-  }
-  x = sx;
-  y = sy;
+  x = msfec_wave::waves_sum<16>(red[0]);
+  y = msfec_wave::waves_sum<16>(red[1]);
 }
 
 constexpr int kCoarseThreads = 1024;
@@ -3137,7 +3129,7 @@ __global__ __launch_bounds__(kCoarseThreads) void coarse_pcg_kernel(
     double* res_out) {
   constexpr int NST = (DIM == 3) ? 27 : 9, CEN = (NST - 1) / 2;
   extern __shared__ double dyn[];
-  __shared__ double red[2][16][2];
+  __shared__ double red[2][2][16];
   const int S = nc + 1, ni = nc - 1;
   const int nnode = (DIM == 3) ? S * S * S : S * S;
   const int nint = (DIM == 3) ? ni * ni * ni : ni * ni;
@@ -3215,14 +3207,157 @@ __global__ __launch_bounds__(kCoarseThreads) void coarse_pcg_kernel(
   }
 }
 
-// The coarse Jacobi-PCG: coarse_pcg_kernel where its LDS holds the grid,
-// the general one-workgroup kernel beyond (its vectors in global memory).
+// The same with up to T nodes per thread (nodes tid, tid + threads, ...), their
+// vectors in registers and only the search direction in LDS.  A single
+// workgroup reads K through one CU: with one node per thread its row stays in
+// registers; with more the entries come from L2 each iteration, nine at a time
+// and one group ahead of their use, which bounds it (216 bytes a node at 64
+// bytes a clock).  A solve of 15^3 nodes takes 0.95 ms, of 7^2 (one wave) 20
+// us; 1.24 ms and 67 us by coarse_pcg_kernel.
+template <int DIM, int T>
+__global__ __launch_bounds__(kCoarseThreads) void coarse_pcg_reg_kernel(
+    int nc, const double* __restrict__ K, const double* __restrict__ rhs, double* __restrict__ u,
+    double abs_tol, double rel_tol, int max_iter, int* iters_out, double* res_out) {
+  constexpr int NST = (DIM == 3) ? 27 : 9, CEN = (NST - 1) / 2, NG = NST / 9;
+  extern __shared__ double P[];
+  __shared__ double red[2][2][16];
+  const int S = nc + 1, ni = nc - 1, nt = blockDim.x, tid = threadIdx.x;
+  const int nnode = (DIM == 3) ? S * S * S : S * S;
+  const int nint = (DIM == 3) ? ni * ni * ni : ni * ni;
+  const __amdgpu_buffer_rsrc_t kb = msfec_wave::buffer_of(K, NST * nnode * 8);
+  for (int i = tid; i < nnode; i += nt) {
+    P[i] = 0.0;
+    u[i] = 0.0;
+  }
+  for (int i = tid; i < 64; i += nt) (&red[0][0][0])[i] = 0.0;
+  int id[T];  // (threads without a node follow the first)
+  double x[T], r[T], di[T], q[T];
+  double bb = 0.0, rz = 0.0;
+  __syncthreads();  // zeroed
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const bool on = tid + t * nt < nint;
+    const int j = on ? tid + t * nt : 0;
+    const int jx = j % ni, jr = j / ni;
+    const int jy = (DIM == 3) ? jr % ni : jr, jz = (DIM == 3) ? jr / ni : 0;
+    id[t] = (jx + 1) + S * (jy + 1) + (DIM == 3 ? S * S * (jz + 1) : 0);
+    x[t] = 0.0;
+    r[t] = on ? rhs[id[t]] : 0.0;
+    di[t] = on ? 1.0 / K[(size_t)CEN * nnode + id[t]] : 0.0;
+    q[t] = di[t] * r[t];
+    if (on) P[id[t]] = q[t];
+    bb = fma(r[t], r[t], bb);
+    rz = fma(r[t], q[t], rz);
+  }
+  auto group = [&](int t, int g, double (&k)[9]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 9; ++e)
+      k[e] = msfec_wave::buffer_f64(kb, id[t] * 8, (g * 9 + e) * nnode * 8);
+  };
+  auto products = [&](int t, int g, const double (&k)[9]) __attribute__((always_inline)) {
+    int at = id[t] + (DIM == 3 ? S * S * (g - 1) : 0);
+    // (hidden: the addresses of all neighbours formed ahead of the iteration
+    // would not fit the registers)
+    asm volatile("" : "+v"(at));
+    double s = 0.0;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) s = fma(k[e], P[at + e % 3 - 1 + S * (e / 3 - 1)], s);
+    return s;
+  };
+  double k[T == 1 ? NG : 2][9];
+  if (T == 1)
+#pragma unroll
+    for (int g = 0; g < NG; ++g) group(0, g, k[g]);
+  coarse_block_sum2(bb, rz, red[0]);  // also: p is in LDS
+  const double stop = fmax(abs_tol * abs_tol, rel_tol * rel_tol * bb);
+  double rr = bb;
+  int it = 0;
+  while (rr > stop && it < max_iter) {
+    double pq = 0.0;
+    if (T > 1) group(0, 0, k[0]);
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      q[t] = 0.0;
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const int n = t * NG + g;
+        if (T > 1 && n + 1 < T * NG) group((n + 1) / NG, (n + 1) % NG, k[(n + 1) & 1]);
+        if (T > 1) __builtin_amdgcn_sched_barrier(0);
+        q[t] += products(t, g, k[T == 1 ? g : n & 1]);
+        if (T > 1) __builtin_amdgcn_sched_barrier(0);
+      }
+      if (tid + t * nt < nint) pq = fma(P[id[t]], q[t], pq);
+    }
+    pq = msfec_wave::wave_sum(pq);
+    if ((tid & 63) == 0) red[1][0][tid >> 6] = pq;
+    __syncthreads();
+    pq = msfec_wave::waves_sum<16>(red[1][0]);
+    if (!(pq > 0.0)) break;  // not SPD: reported as not converged
+    const double alpha = rz / pq;
+    double rz1 = 0.0;
+    rr = 0.0;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const bool on = tid + t * nt < nint;
+      x[t] = fma(alpha, P[id[t]], x[t]);
+      r[t] = on ? fma(-alpha, q[t], r[t]) : 0.0;
+      q[t] = di[t] * r[t];
+      rz1 = fma(r[t], q[t], rz1);
+      rr = fma(r[t], r[t], rr);
+    }
+    coarse_block_sum2(rz1, rr, red[0]);  // also: every thread is done reading p
+    const double beta = rz1 / rz;
+    rz = rz1;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const double v = fma(beta, P[id[t]], q[t]);
+      if (tid + t * nt < nint) P[id[t]] = v;
+    }
+    __syncthreads();
+    ++it;
+  }
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+    if (tid + t * nt < nint) u[id[t]] = x[t];
+  if (tid == 0) {
+    *iters_out = (rr > stop) ? -it : it;
+    *res_out = sqrt(rr);
+  }
+}
+
+template <int DIM, int T>
+hipError_t launch_coarse_reg(int nc, const double* K, const double* rhs, double* u, double abs_tol,
+                             double rel_tol, int max_iter, int* iters, double* res, hipStream_t s) {
+  size_t nnode = 1, nint = 1;
+  for (int d = 0; d < DIM; ++d) {
+    nnode *= (size_t)(nc + 1);
+    nint *= (size_t)(nc - 1);
+  }
+  const unsigned nt = (unsigned)(((nint + T - 1) / T + 63) / 64 * 64);
+  hipLaunchKernelGGL((coarse_pcg_reg_kernel<DIM, T>), dim3(1), dim3(nt), nnode * sizeof(double), s,
+                     nc, K, rhs, u, abs_tol, rel_tol, max_iter, iters, res);
+  return hipGetLastError();
+}
+
+// The coarse Jacobi-PCG: with its vectors in registers up to 4 nodes per
+// thread, coarse_pcg_kernel where its LDS holds the grid, the general
+// one-workgroup kernel beyond (its vectors in global memory).
 // Buffers as coarse_cg_kernel's (pv holds the inverse diagonal in the former).
 hipError_t launch_coarse_cg(int dim, int nc, const double* K, const double* rhs, double* u,
                             double* r, double* z, double* pv, double* qv, double abs_tol,
                             double rel_tol, int max_iter, int* iters, double* res,
                             hipStream_t s) {
   const size_t lds = coarse_pcg_lds(dim, nc);
+  size_t nint = 1;
+  for (int d = 0; d < dim; ++d) nint *= (size_t)(nc > 1 ? nc - 1 : 0);
+  if (nint > 0 && nint <= 4 * kCoarseThreads) {
+    const bool one = nint <= kCoarseThreads;
+    if (dim == 3)
+      return one ? launch_coarse_reg<3, 1>(nc, K, rhs, u, abs_tol, rel_tol, max_iter, iters, res, s)
+                 : launch_coarse_reg<3, 4>(nc, K, rhs, u, abs_tol, rel_tol, max_iter, iters, res, s);
+    return one ? launch_coarse_reg<2, 1>(nc, K, rhs, u, abs_tol, rel_tol, max_iter, iters, res, s)
+               : launch_coarse_reg<2, 4>(nc, K, rhs, u, abs_tol, rel_tol, max_iter, iters, res, s);
+  }
   if (nc >= 2 && lds <= 150 * 1024) {
     const void* fn = (dim == 3) ? (const void*)coarse_pcg_kernel<3> : (const void*)coarse_pcg_kernel<2>;
     if (lds > 48 * 1024) {

@@ -13,6 +13,8 @@ using msfec_detail::Q1tBasis;
 using msfec_detail::Q1tCg;
 using msfec_detail::Q1tRows;
 using msfec_wave::block_sums;
+using msfec_wave::buffer_f64;
+using msfec_wave::buffer_of;
 using msfec_wave::from_left;
 using msfec_wave::from_right;
 using msfec_wave::wave_sum;
@@ -178,15 +180,6 @@ __global__ __launch_bounds__(RowTile<M>::NT, 2) void q1t_rows_kernel(Q1tRows g) 
     if (n < g.nr) g.rhs[((size_t)cell * g.nr + n) * M3 + node] = rh[n];
 }
 
-// Entry at byte offset `lane` (per lane) + `uni` (uniform) of the rows of one
-// cell, as a buffer load: with plain pointers the compiler forms a 64-bit
-// address per lane for every entry ahead of the loop, and spills them.
-typedef unsigned row_v2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ double row_entry(__amdgpu_buffer_rsrc_t rsrc, int lane, int uni) {
-  const row_v2 t = __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane, uni, 0);
-  return __hiloint2double((int)t.y, (int)t.x);
-}
-
 // Jacobi-preconditioned conjugate gradients, one right-hand side of one
 // coarse cell per workgroup, LZ nodes of a column in z per thread.  x, r and p
 // stay in registers; p is in LDS as well, flat and padded with zeros, so that
@@ -219,7 +212,7 @@ __global__ __launch_bounds__(M * M * M / LZ < 64 ? 64 : M * M * M / LZ) void q1t
   const int row0 = k0 * M2 + col;
   const double* st = g.st + (size_t)cell * 15 * M3;
   const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(st), 0, 15 * M3 * 8, 0x00027000);
+      buffer_of(st, 15 * M3 * 8);
   for (int i = tid; i < M3 + 2 * PAD; i += NT) P[i] = 0.0;
   for (int i = tid; i < M3 + M; i += NT) UM[i] = UP[i] = 0.0;
   for (int i = tid; i < NS * M2 + M; i += NT) BM[i] = BP[i] = 0.0;
@@ -229,7 +222,7 @@ __global__ __launch_bounds__(M * M * M / LZ < 64 ? 64 : M * M * M / LZ) void q1t
   for (int z = 0; z < LZ; ++z) {
     x[z] = 0.0;
     r[z] = g.rhs[((size_t)cell * g.nr + n) * M3 + row0 + z * M2];
-    p[z] = row_entry(rsrc, row0 * 8, (14 * M3 + z * M2) * 8) * r[z];
+    p[z] = buffer_f64(rsrc, row0 * 8, (14 * M3 + z * M2) * 8) * r[z];
     rz = fma(r[z], p[z], rz);
     rr = fma(r[z], r[z], rr);
   }
@@ -266,7 +259,7 @@ __global__ __launch_bounds__(M * M * M / LZ < 64 ? 64 : M * M * M / LZ) void q1t
     auto fetch = [&](int gr) {
 #pragma unroll
       for (int t = 0; t < (gr & 1 ? 5 : 9); ++t)
-        at[gr % 3][t] = row_entry(rsrc, row0 * 8, (((gr & 1 ? 9 : 0) + t) * M3 + (gr >> 1) * M2) * 8);
+        at[gr % 3][t] = buffer_f64(rsrc, row0 * 8, (((gr & 1 ? 9 : 0) + t) * M3 + (gr >> 1) * M2) * 8);
     };
     fetch(0);
     fetch(1);
@@ -328,7 +321,7 @@ __global__ __launch_bounds__(M * M * M / LZ < 64 ? 64 : M * M * M / LZ) void q1t
     double rz1 = 0.0, dv[LZ];
     rr = 0.0;
 #pragma unroll
-    for (int z = 0; z < LZ; ++z) dv[z] = row_entry(rsrc, row0 * 8, (14 * M3 + z * M2) * 8);
+    for (int z = 0; z < LZ; ++z) dv[z] = buffer_f64(rsrc, row0 * 8, (14 * M3 + z * M2) * 8);
 #pragma unroll
     for (int z = 0; z < LZ; ++z) {
       x[z] = fma(alpha, p[z], x[z]);

@@ -182,8 +182,7 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
     for (int d = 0; d < 3; ++d) tim[d * M + tid] = 1.0 / (mf[d] * t);
   }
   const int at0 = (k0 * S + j) * S + i;  // lattice point of the first cell
-  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      g.MF + (size_t)cell * 22 * M3, 0, 22 * M3 * 8, 0x00027000);
+  const __amdgpu_buffer_rsrc_t rsrc = msfec_wave::buffer_of(g.MF + (size_t)cell * 22 * M3, 22 * M3 * 8);
   const int lane0 = (k0 * M2 + col) * 16;
   auto pair = [&](int e, int t) {
     const mass_v4 m = __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane0, (e * M3 + t * M2) * 16, 0);

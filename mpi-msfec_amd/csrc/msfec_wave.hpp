@@ -1,8 +1,22 @@
-// Lane shifts, and sums over a wave and a workgroup.
+// Buffer loads, lane shifts, and sums over a wave and a workgroup.
 #pragma once
 #include <hip/hip_runtime.h>
 
 namespace msfec_wave {
+
+// `bytes` bytes at p, the same for all lanes, for buffer loads: a load outside
+// of them returns zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const double* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(p), 0, bytes, 0x00027000);
+}
+// The value at byte offset `lane` (per lane) + `uni` (uniform).  With plain
+// pointers the compiler forms a 64-bit address per lane for every load of an
+// unrolled loop ahead of it, and spills them.
+typedef unsigned buffer_v2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ double buffer_f64(__amdgpu_buffer_rsrc_t b, int lane, int uni) {
+  const buffer_v2 t = __builtin_amdgcn_raw_buffer_load_b64(b, lane, uni, 0);
+  return __hiloint2double((int)t.y, (int)t.x);
+}
 
 // Sum over the N lanes (a power of two, at most 16) of a row, or of N values
 // that repeat within it: every lane has it, in the same bits, as a + b = b + a.
