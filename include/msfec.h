@@ -62,8 +62,10 @@ enum { MSFEC_RHS_CONST = 0, MSFEC_RHS_CELL = 1, MSFEC_RHS_QP = 2 };
 enum { MSFEC_REACTION_NONE = 0, MSFEC_REACTION_CONST = 1, MSFEC_REACTION_CELL = 2 };
 /* local solver: banded Cholesky of the interior system, the analogue of
  * use_direct_solver_basis = true (source/Q/q_basis.cc:304-330):
- *   BAND_FP64      FP64, one pivot per step on the vector ALUs (the default
- *                  of the Python and C++ front ends);
+ *   BAND_FP64      as BAND_FP64_MFMA, and the cells that are not positive
+ *                  definite again with one pivot per step on the vector ALUs,
+ *                  which takes pivots of either sign (the default of the
+ *                  Python and C++ front ends);
  *   BAND_FP64_MFMA FP64, four pivots per step with FP64 matrix-core updates;
  *   BAND_MIXED     FP32 factor on the matrix cores and iterative refinement
  *                  with the residual in FP64: a cell stops refining once the

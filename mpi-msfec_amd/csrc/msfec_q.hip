@@ -357,6 +357,7 @@ struct BandArgs {
   double* M;     // [cell][nv][nv]
   double* bvec;  // [cell][nv]
   int* status;   // [cell]
+  int failed_only;  // q_band_kernel: only the cells whose status is not OK
 };
 
 template <int DIM>
@@ -1027,6 +1028,7 @@ __global__ __launch_bounds__(64, 2) void q_band_kernel(BandArgs a) {
   using D = Dirs<DIM>;
   const int cell = blockIdx.x;
   const int lane = threadIdx.x;
+  if (a.failed_only && a.status[cell] == MSFEC_CELL_OK) return;
   __shared__ BandSmem sh;
   extern __shared__ double dyn[];  // fast path: fine-cell coefficient | reaction | load
   const double* cf = dyn;
@@ -4969,19 +4971,26 @@ msfec_status msfec_q_compute(msfec_q_handle h, void* stream) {
       else
         hipLaunchKernelGGL((q_blk_refine_kernel<2>), dim3(h->n_cells), dim3(64), 0, s, a);
     }
-  } else if (mfma && fast) {
-    launch_factor64(c.dim, c.nt, h->n_cells, s, a);
-  } else if (mfma) {
-    // tensor coefficients: stencil tables of q_assemble_kernel
-    if (c.dim == 3) LAUNCH_BAND(q_band_mfma_kernel, 3, false);
-    else LAUNCH_BAND(q_band_mfma_kernel, 2, false);
   } else {
-    if (c.dim == 3) {
-      if (fast) LAUNCH_BAND(q_band_kernel, 3, true);
-      else LAUNCH_BAND(q_band_kernel, 3, false);
-    } else {
-      if (fast) LAUNCH_BAND(q_band_kernel, 2, true);
-      else LAUNCH_BAND(q_band_kernel, 2, false);
+    // FP64 on the matrix cores.  BAND_FP64 as well, and then its one-pivot
+    // kernel for the cells that are not positive definite: it carries on with
+    // pivots of either sign (a reaction rate below zero) and tells which of
+    // the non-finite values came first.  For all cells that kernel takes twice
+    // the time at every size (a pass of 125 cells of 8^3 458 against 230 us, of
+    // 4096 1775 and 904; 64 of 32^2 1130 and 552, 1024 of 2^2 62 and 47).
+    if (fast) launch_factor64(c.dim, mfma ? c.nt : band_tile_rows(h->bw, h->p.band_window), h->n_cells, s, a);
+    else if (c.dim == 3) LAUNCH_BAND(q_band_mfma_kernel, 3, false);
+    else LAUNCH_BAND(q_band_mfma_kernel, 2, false);
+    if (!mfma) {
+      MSFEC_HIP(hipGetLastError());
+      a.failed_only = 1;
+      if (c.dim == 3) {
+        if (fast) LAUNCH_BAND(q_band_kernel, 3, true);
+        else LAUNCH_BAND(q_band_kernel, 3, false);
+      } else {
+        if (fast) LAUNCH_BAND(q_band_kernel, 2, true);
+        else LAUNCH_BAND(q_band_kernel, 2, false);
+      }
     }
   }
 #undef LAUNCH_BAND
