@@ -50,7 +50,8 @@ extern thread_local std::string g_last_error;
 size_t band_ldl_panel_doubles(int n);
 size_t band_ldl_z_doubles(int n);
 hipError_t band_ldl_solve(int n_cells, int n, int bw, const double* rows, const int* loff,
-                          double* pan, double* zst, double* X, int* status, hipStream_t s);
+                          double* pan, double* zst, double* X, int* status, bool failed_only,
+                          hipStream_t s);
 // the same with an FP32 factor and FP64 refinement (msfec_q.hip)
 size_t band_ldl_mixed_doubles(int n);
 std::vector<int> band_upper_table(const std::vector<int>& loff, int n);
@@ -834,7 +835,7 @@ msfec_status msfec_ned_compute(msfec_ned_handle h, void* stream) {
                                                h->d_mixed, h->d_status, h->prm.max_refine, s));
   else
     NED_HIP(msfec_detail::band_ldl_solve(h->n_cells, h->conf.n, h->conf.p, h->d_rows, h->d_loff,
-                                         h->d_pan, h->d_zst, h->d_X, h->d_status, s));
+                                         h->d_pan, h->d_zst, h->d_X, h->d_status, false, s));
   if (ev) NED_HIP(hipEventRecord((*ev)[2], s));
   hipLaunchKernelGGL(ned_element_kernel, dim3(h->n_cells), dim3(kNThreads), elem_lds, s, a);
   NED_HIP(hipGetLastError());

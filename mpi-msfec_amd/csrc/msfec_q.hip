@@ -357,7 +357,7 @@ struct BandArgs {
   double* M;     // [cell][nv][nv]
   double* bvec;  // [cell][nv]
   int* status;   // [cell]
-  int failed_only;  // q_band_kernel: only the cells whose status is not OK
+  int failed_only;  // q_band_kernel, LDL^T: only the cells whose status is not OK
 };
 
 template <int DIM>
@@ -2304,6 +2304,7 @@ __global__ __launch_bounds__(64, BkOcc<R>::waves) void q_blk_factor_kernel(BandA
   typedef typename Mf<R>::v4 V4;
   const int cell = blockIdx.x;
   const int lane = threadIdx.x;
+  if (LDL && a.failed_only && a.status[cell] == MSFEC_CELL_OK) return;
   __shared__ BandSmem sh;
   __shared__ BkSmem<R> ms;
   int my_off = 0;
@@ -4146,9 +4147,11 @@ size_t band_ldl_z_doubles(int n) { return (size_t)panel_quads(n) * 32; }
 // The matrix-core band LDL^T of the Q_Ned interior systems: rows
 // [cells][n][24] (16 lower entries, diagonal first, with their offsets in
 // loff [n][16]; 8 right-hand sides), the solutions to X [cells][n][8], the
-// cell status (MSFEC_CELL_NOT_SPD for a zero pivot) to status.
+// cell status (MSFEC_CELL_NOT_SPD for a zero pivot) to status.  failed_only:
+// only the cells whose status is not MSFEC_CELL_OK.
 hipError_t band_ldl_solve(int n_cells, int n, int bw, const double* rows, const int* loff,
-                          double* pan, double* zst, double* X, int* status, hipStream_t s) {
+                          double* pan, double* zst, double* X, int* status, bool failed_only,
+                          hipStream_t s) {
   const int nt = band_tile_rows(bw, 0);
   if (nt == 0) return hipErrorInvalidValue;
   BandArgs a{};
@@ -4160,6 +4163,7 @@ hipError_t band_ldl_solve(int n_cells, int n, int bw, const double* rows, const 
   a.zst = zst;
   a.X = X;
   a.status = status;
+  a.failed_only = failed_only;
 #define LDL(NT) \
   hipLaunchKernelGGL((q_blk_factor_kernel<double, 2, BK_X0, true, NT>), dim3(n_cells), dim3(64), 0, s, a)
   if (nt == 1) LDL(1);

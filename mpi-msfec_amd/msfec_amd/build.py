@@ -13,7 +13,7 @@ INCLUDE = os.path.join(REPO, "include")
 LIB = os.path.join(HERE, "libmsfec_hip.so")
 
 SOURCES = ["msfec_q.hip", "msfec_ned.hip", "msfec_rt.hip", "msfec_uneven.hip", "msfec_nrt.hip",
-           "msfec_nrt_seq.hip", "msfec_q1t.hip", "msfec_rt3_proj.hip"]
+           "msfec_nrt_seq.hip", "msfec_q1t.hip", "msfec_rt3_proj.hip", "msfec_lines.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
