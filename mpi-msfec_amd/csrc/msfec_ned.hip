@@ -639,21 +639,23 @@ void ned_free(msfec_ned_batch* h) {
 
 // Copied on the handle's stream (that of its last compute call), waited for:
 // work still in flight there reads the old buffer to the end.
-msfec_status ned_in(hipStream_t s, double* dst, const double* src, size_t count, int loc) {
+msfec_status ned_in(hipStream_t s, double* dst, const double* src, size_t count, int loc,
+                    bool wait = true) {
   if (!src) return ned_fail(MSFEC_ERR_INVALID, "null data pointer");
   NED_HIP(hipMemcpyAsync(dst, src, count * sizeof(double),
                          loc == MSFEC_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-  NED_HIP(hipStreamSynchronize(s));
+  if (wait) NED_HIP(hipStreamSynchronize(s));
   return MSFEC_OK;
 }
 
 // Copied on the handle's stream and waited for: a device destination holds
 // the data when the call returns (a device-to-device hipMemcpy may return first).
-msfec_status ned_out(hipStream_t s, double* dst, const double* src, size_t count, int loc) {
+msfec_status ned_out(hipStream_t s, double* dst, const double* src, size_t count, int loc,
+                     bool wait = true) {
   if (!dst) return ned_fail(MSFEC_ERR_INVALID, "null output pointer");
   NED_HIP(hipMemcpyAsync(dst, src, count * sizeof(double),
                          loc == MSFEC_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
-  NED_HIP(hipStreamSynchronize(s));
+  if (wait) NED_HIP(hipStreamSynchronize(s));
   return MSFEC_OK;
 }
 
@@ -798,10 +800,11 @@ msfec_status msfec_ned_set_coefficients(msfec_ned_handle h, const double* a, con
   if (!h) return ned_fail(MSFEC_ERR_INVALID, "null handle");
   if (loc != MSFEC_HOST && loc != MSFEC_DEVICE) return ned_fail(MSFEC_ERR_INVALID, "bad location");
   const size_t cnt = (size_t)h->n_cells * h->conf.m * h->conf.m;
-  msfec_status st = ned_in(h->stream, h->d_a, a, cnt, loc);
-  if (st == MSFEC_OK) st = ned_in(h->stream, h->d_binv, binv, cnt, loc);
-  if (st == MSFEC_OK) st = ned_in(h->stream, h->d_r, r, cnt, loc);
-  if (st == MSFEC_OK) st = ned_in(h->stream, h->d_f, f, 2 * cnt, loc);
+  msfec_status st = ned_in(h->stream, h->d_a, a, cnt, loc, false);
+  if (st == MSFEC_OK) st = ned_in(h->stream, h->d_binv, binv, cnt, loc, false);
+  if (st == MSFEC_OK) st = ned_in(h->stream, h->d_r, r, cnt, loc, false);
+  if (st == MSFEC_OK) st = ned_in(h->stream, h->d_f, f, 2 * cnt, loc, false);
+  NED_HIP(hipStreamSynchronize(h->stream));
   if (st != MSFEC_OK) return st;
   h->coef_set = true;
   return MSFEC_OK;
@@ -853,17 +856,16 @@ msfec_status msfec_ned_synchronize(msfec_ned_handle h) {
 msfec_status msfec_ned_get_element(msfec_ned_handle h, double* M, double* b, int loc) {
   if (!h) return ned_fail(MSFEC_ERR_INVALID, "null handle");
   if (!h->computed) return ned_fail(MSFEC_ERR_STATE, "compute not called");
-  NED_HIP(hipStreamSynchronize(h->stream));
   msfec_status st = MSFEC_OK;
-  if (M) st = ned_out(h->stream, M, h->d_M, (size_t)h->n_cells * 64, loc);
-  if (st == MSFEC_OK && b) st = ned_out(h->stream, b, h->d_b, (size_t)h->n_cells * kNR, loc);
+  if (M) st = ned_out(h->stream, M, h->d_M, (size_t)h->n_cells * 64, loc, false);
+  if (st == MSFEC_OK && b) st = ned_out(h->stream, b, h->d_b, (size_t)h->n_cells * kNR, loc, false);
+  NED_HIP(hipStreamSynchronize(h->stream));
   return st;
 }
 
 msfec_status msfec_ned_get_basis(msfec_ned_handle h, double* Psi, int loc) {
   if (!h) return ned_fail(MSFEC_ERR_INVALID, "null handle");
   if (!h->computed) return ned_fail(MSFEC_ERR_STATE, "compute not called");
-  NED_HIP(hipStreamSynchronize(h->stream));
   return ned_out(h->stream, Psi, h->d_psi, (size_t)h->n_cells * kNR * h->conf.N, loc);
 }
 

@@ -2522,19 +2522,21 @@ void nrt_free(msfec_nrt_batch* h) {
 }
 
 // Copied on the handle's stream (that of its last compute call), waited for.
-msfec_status nrt_in(hipStream_t s, void* dst, const void* src, size_t bytes, int loc) {
+msfec_status nrt_in(hipStream_t s, void* dst, const void* src, size_t bytes, int loc,
+                    bool wait = true) {
   NRT_HIP(hipMemcpyAsync(dst, src, bytes,
                          loc == MSFEC_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-  NRT_HIP(hipStreamSynchronize(s));
+  if (wait) NRT_HIP(hipStreamSynchronize(s));
   return MSFEC_OK;
 }
 
-msfec_status nrt_out(hipStream_t s, double* dst, const double* src, size_t count, int loc) {
+msfec_status nrt_out(hipStream_t s, double* dst, const double* src, size_t count, int loc,
+                     bool wait = true) {
   if (!dst) return nrt_fail(MSFEC_ERR_INVALID, "null output pointer");
   if (loc != MSFEC_HOST && loc != MSFEC_DEVICE) return nrt_fail(MSFEC_ERR_INVALID, "bad location");
   NRT_HIP(hipMemcpyAsync(dst, src, count * sizeof(double),
                          loc == MSFEC_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
-  NRT_HIP(hipStreamSynchronize(s));
+  if (wait) NRT_HIP(hipStreamSynchronize(s));
   return MSFEC_OK;
 }
 
@@ -2764,10 +2766,11 @@ msfec_status msfec_nrt_set_coefficients(msfec_nrt_handle h, const double* ainv, 
   if (!h || !ainv || !b) return nrt_fail(MSFEC_ERR_INVALID, "null argument");
   if (loc != MSFEC_HOST && loc != MSFEC_DEVICE) return nrt_fail(MSFEC_ERR_INVALID, "bad location");
   const size_t pts = (size_t)h->n_cells * ((size_t)1 << (3 * h->l)) * 8;
-  msfec_status st = nrt_in(h->stream, h->d_ainv, ainv, pts * 6 * sizeof(double), loc);
-  if (st == MSFEC_OK) st = nrt_in(h->stream, h->d_b, b, pts * sizeof(double), loc);
-  if (st == MSFEC_OK && r) st = nrt_in(h->stream, h->d_r, r, pts * sizeof(double), loc);
-  if (st == MSFEC_OK && f) st = nrt_in(h->stream, h->d_f, f, pts * 3 * sizeof(double), loc);
+  msfec_status st = nrt_in(h->stream, h->d_ainv, ainv, pts * 6 * sizeof(double), loc, false);
+  if (st == MSFEC_OK) st = nrt_in(h->stream, h->d_b, b, pts * sizeof(double), loc, false);
+  if (st == MSFEC_OK && r) st = nrt_in(h->stream, h->d_r, r, pts * sizeof(double), loc, false);
+  if (st == MSFEC_OK && f) st = nrt_in(h->stream, h->d_f, f, pts * 3 * sizeof(double), loc, false);
+  NRT_HIP(hipStreamSynchronize(h->stream));
   if (st != MSFEC_OK) return st;
   h->has_r = r != nullptr;
   h->has_f = f != nullptr;
@@ -2854,8 +2857,9 @@ msfec_status msfec_nrt_get_element(msfec_nrt_handle h, double* M, double* b, int
   if (!h) return nrt_fail(MSFEC_ERR_INVALID, "null handle");
   if (!h->computed) return nrt_fail(MSFEC_ERR_STATE, "compute not called");
   msfec_status st = MSFEC_OK;
-  if (M) st = nrt_out(h->stream, M, h->d_M, (size_t)h->n_cells * kNB * kNB, loc);
-  if (st == MSFEC_OK && b) st = nrt_out(h->stream, b, h->d_rhs, (size_t)h->n_cells * kNB, loc);
+  if (M) st = nrt_out(h->stream, M, h->d_M, (size_t)h->n_cells * kNB * kNB, loc, false);
+  if (st == MSFEC_OK && b) st = nrt_out(h->stream, b, h->d_rhs, (size_t)h->n_cells * kNB, loc, false);
+  NRT_HIP(hipStreamSynchronize(h->stream));
   return st;
 }
 
@@ -3135,8 +3139,9 @@ msfec_status msfec_rt3_set_coefficients(msfec_rt3_handle h, const double* ainv, 
   if (!h || !ainv) return nrt_fail(MSFEC_ERR_INVALID, "null argument");
   if (loc != MSFEC_HOST && loc != MSFEC_DEVICE) return nrt_fail(MSFEC_ERR_INVALID, "bad location");
   const size_t pts = (size_t)h->n_cells * ((size_t)1 << (3 * h->l)) * 8;
-  msfec_status st = nrt_in(h->stream, h->d_ainv, ainv, pts * 6 * sizeof(double), loc);
-  if (st == MSFEC_OK && f) st = nrt_in(h->stream, h->d_f, f, pts * sizeof(double), loc);
+  msfec_status st = nrt_in(h->stream, h->d_ainv, ainv, pts * 6 * sizeof(double), loc, false);
+  if (st == MSFEC_OK && f) st = nrt_in(h->stream, h->d_f, f, pts * sizeof(double), loc, false);
+  NRT_HIP(hipStreamSynchronize(h->stream));
   if (st != MSFEC_OK) return st;
   h->has_f = f != nullptr;
   h->coef_set = true;
@@ -3181,8 +3186,9 @@ msfec_status msfec_rt3_get_element(msfec_rt3_handle h, double* M, double* b, int
   if (!h) return nrt_fail(MSFEC_ERR_INVALID, "null handle");
   if (!h->computed) return nrt_fail(MSFEC_ERR_STATE, "compute not called");
   msfec_status st = MSFEC_OK;
-  if (M) st = nrt_out(h->stream, M, h->d_M, (size_t)h->n_cells * 49, loc);
-  if (st == MSFEC_OK && b) st = nrt_out(h->stream, b, h->d_b, (size_t)h->n_cells * 7, loc);
+  if (M) st = nrt_out(h->stream, M, h->d_M, (size_t)h->n_cells * 49, loc, false);
+  if (st == MSFEC_OK && b) st = nrt_out(h->stream, b, h->d_b, (size_t)h->n_cells * 7, loc, false);
+  NRT_HIP(hipStreamSynchronize(h->stream));
   return st;
 }
 

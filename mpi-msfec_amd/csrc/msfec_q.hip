@@ -4395,10 +4395,12 @@ msfec_status copy_in(hipStream_t s, double* dst, const double* src, size_t count
 // Outputs are copied on the handle's stream and waited for: a device
 // destination holds the data when the call returns, whatever stream the
 // caller reads it on next (a device-to-device hipMemcpy may return first).
-msfec_status copy_out(hipStream_t s, double* dst, const double* src, size_t count, int loc) {
+// With `wait` off the call returns before (a later one on the stream waits).
+msfec_status copy_out(hipStream_t s, double* dst, const double* src, size_t count, int loc,
+                      bool wait = true) {
   MSFEC_HIP(hipMemcpyAsync(dst, src, count * sizeof(double),
                            loc == MSFEC_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
-  MSFEC_HIP(hipStreamSynchronize(s));
+  if (wait) MSFEC_HIP(hipStreamSynchronize(s));
   return MSFEC_OK;
 }
 
@@ -5055,23 +5057,22 @@ msfec_status msfec_q_kernel_times(msfec_q_handle h, float* ms, int max, int* n) 
 msfec_status msfec_q_get_element(msfec_q_handle h, double* M, double* b, int loc) {
   if (!h) return fail(MSFEC_ERR_INVALID, "null handle");
   if (!h->computed) return fail(MSFEC_ERR_STATE, "compute not called");
-  MSFEC_HIP(hipStreamSynchronize(h->stream));
   const size_t nv = h->conf.nv;
   if (M) {
-    msfec_status st = copy_out(h->stream, M, h->d_M, (size_t)h->n_cells * nv * nv, loc);
+    msfec_status st = copy_out(h->stream, M, h->d_M, (size_t)h->n_cells * nv * nv, loc, false);
     if (st) return st;
   }
   if (b) {
-    msfec_status st = copy_out(h->stream, b, h->d_b, (size_t)h->n_cells * nv, loc);
+    msfec_status st = copy_out(h->stream, b, h->d_b, (size_t)h->n_cells * nv, loc, false);
     if (st) return st;
   }
+  MSFEC_HIP(hipStreamSynchronize(h->stream));
   return MSFEC_OK;
 }
 
 msfec_status msfec_q_get_basis(msfec_q_handle h, double* Psi, int loc) {
   if (!h || !Psi) return fail(MSFEC_ERR_INVALID, "null argument");
   if (!h->computed) return fail(MSFEC_ERR_STATE, "compute not called");
-  MSFEC_HIP(hipStreamSynchronize(h->stream));
   return copy_out(h->stream, Psi, h->d_psi, (size_t)h->n_cells * h->conf.nv * h->conf.nn, loc);
 }
 
@@ -5149,21 +5150,21 @@ msfec_status msfec_coarse_solve(msfec_q_handle h, int nc, double abs_tol, double
                                               h->d_cvec, h->d_cit, abs_tol, rel_tol, max_iter,
                                               h->stream));
   const int nw = h->n_cells * nv;
-  MSFEC_HIP(hipStreamSynchronize(h->stream));
   int it = 0;
   double rr = 0.0;
-  MSFEC_HIP(hipMemcpy(&it, h->d_cit, sizeof(int), hipMemcpyDeviceToHost));
-  MSFEC_HIP(hipMemcpy(&rr, res, sizeof(double), hipMemcpyDeviceToHost));
-  if (iterations) *iterations = it;
-  if (residual) *residual = rr;
   if (u) {
-    msfec_status st = copy_out(h->stream, u, du, nnode, u_loc);
+    msfec_status st = copy_out(h->stream, u, du, nnode, u_loc, false);
     if (st) return st;
   }
   if (weights) {
-    msfec_status st = copy_out(h->stream, weights, dw, (size_t)nw, weights_loc);
+    msfec_status st = copy_out(h->stream, weights, dw, (size_t)nw, weights_loc, false);
     if (st) return st;
   }
+  MSFEC_HIP(hipMemcpyAsync(&it, h->d_cit, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  MSFEC_HIP(hipMemcpyAsync(&rr, res, sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  MSFEC_HIP(hipStreamSynchronize(h->stream));
+  if (iterations) *iterations = it;
+  if (residual) *residual = rr;
   if (it < 0) return fail(MSFEC_ERR_CELL, "coarse CG did not converge");
   return MSFEC_OK;
 }

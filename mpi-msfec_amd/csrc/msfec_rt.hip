@@ -478,20 +478,22 @@ void rt_free(msfec_rt_batch* h) {
 
 // Copied on the handle's stream (that of its last compute call), waited for:
 // work still in flight there reads the old buffer to the end.
-msfec_status rt_in(hipStream_t s, double* dst, const double* src, size_t count, int loc) {
+msfec_status rt_in(hipStream_t s, double* dst, const double* src, size_t count, int loc,
+                   bool wait = true) {
   RT_HIP(hipMemcpyAsync(dst, src, count * sizeof(double),
                         loc == MSFEC_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-  RT_HIP(hipStreamSynchronize(s));
+  if (wait) RT_HIP(hipStreamSynchronize(s));
   return MSFEC_OK;
 }
 
 // Copied on the handle's stream and waited for: a device destination holds
 // the data when the call returns (a device-to-device hipMemcpy may return first).
-msfec_status rt_out(hipStream_t s, double* dst, const double* src, size_t count, int loc) {
+msfec_status rt_out(hipStream_t s, double* dst, const double* src, size_t count, int loc,
+                    bool wait = true) {
   if (!dst) return rt_fail(MSFEC_ERR_INVALID, "null output pointer");
   RT_HIP(hipMemcpyAsync(dst, src, count * sizeof(double),
                         loc == MSFEC_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
-  RT_HIP(hipStreamSynchronize(s));
+  if (wait) RT_HIP(hipStreamSynchronize(s));
   return MSFEC_OK;
 }
 
@@ -615,10 +617,10 @@ msfec_status msfec_rt_set_coefficients(msfec_rt_handle h, const double* a, const
   if (loc != MSFEC_HOST && loc != MSFEC_DEVICE) return rt_fail(MSFEC_ERR_INVALID, "bad location");
   const size_t cnt = (size_t)h->n_cells * h->m * h->m;
   const size_t acnt = cnt * (h->prm.coef_mode == MSFEC_COEF_TENSOR_QP ? 12 : 1);
-  msfec_status st = rt_in(h->stream, h->d_a, a, acnt, loc);
+  msfec_status st = rt_in(h->stream, h->d_a, a, acnt, loc, false);
   if (st != MSFEC_OK) return st;
   if (f) {
-    st = rt_in(h->stream, h->d_f, f, cnt, loc);
+    st = rt_in(h->stream, h->d_f, f, cnt, loc);  // waits for both
   } else {
     const std::vector<double> ones(cnt, 1.0);
     st = rt_in(h->stream, h->d_f, ones.data(), cnt, MSFEC_HOST);
@@ -685,17 +687,16 @@ msfec_status msfec_rt_synchronize(msfec_rt_handle h) {
 msfec_status msfec_rt_get_element(msfec_rt_handle h, double* M, double* b, int loc) {
   if (!h) return rt_fail(MSFEC_ERR_INVALID, "null handle");
   if (!h->computed) return rt_fail(MSFEC_ERR_STATE, "compute not called");
-  RT_HIP(hipStreamSynchronize(h->stream));
   msfec_status st = MSFEC_OK;
-  if (M) st = rt_out(h->stream, M, h->d_M, (size_t)h->n_cells * kNE, loc);
-  if (st == MSFEC_OK && b) st = rt_out(h->stream, b, h->d_b, (size_t)h->n_cells * 5, loc);
+  if (M) st = rt_out(h->stream, M, h->d_M, (size_t)h->n_cells * kNE, loc, false);
+  if (st == MSFEC_OK && b) st = rt_out(h->stream, b, h->d_b, (size_t)h->n_cells * 5, loc, false);
+  RT_HIP(hipStreamSynchronize(h->stream));
   return st;
 }
 
 msfec_status msfec_rt_get_basis(msfec_rt_handle h, double* sigma, int loc) {
   if (!h) return rt_fail(MSFEC_ERR_INVALID, "null handle");
   if (!h->computed) return rt_fail(MSFEC_ERR_STATE, "compute not called");
-  RT_HIP(hipStreamSynchronize(h->stream));
   return rt_out(h->stream, sigma, h->d_sigma, (size_t)h->n_cells * kNB * h->ne, loc);
 }
 
