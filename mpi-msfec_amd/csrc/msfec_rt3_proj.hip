@@ -12,7 +12,7 @@
 // (msfec_trig.hpp): z^ = Mf^-1 (r^ - kappa s), kappa . z^ = 0, at
 // the cost of 36 LDS passes over a component.
 // 64 cells of 16^3 with the coefficients of the reference example: 49
-// iterations and 3.5 ms, against 180 and 30.4 ms on the curl-curl system with
+// iterations and 3.2 ms, against 180 and 30.4 ms on the curl-curl system with
 // its vectors in memory.
 //
 // Cells whose A^-1 is not positive definite or not finite, or whose contrast
@@ -27,6 +27,7 @@ namespace {
 
 using msfec_detail::Rt3Proj;
 using msfec_wave::block_sums;
+using msfec_wave::buffer_f64;
 using msfec_wave::from_left;
 using msfec_wave::from_right;
 using msfec_wave::wave_sum;
@@ -193,7 +194,15 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
     const double t = lev * (1.0 / M);
     return d == (nb >> 1) ? ((nb & 1) ? t : 1.0 - t) * (1.0 / M2) : 0.0;
   };
-  double x[3][LZ], r[3][LZ], p[3][LZ];
+  double r[3][LZ], p[3][LZ];
+  // x waits at the place of its faces in g.S: it is touched once an iteration,
+  // and its 3 LZ values would not fit the registers (240 of them in scratch at
+  // M = 16; a pass of 64 cells took 3.53 ms with it there and 3.20 ms so)
+  double* out = g.S + ((size_t)cell * 6 + nb) * 3 * C::NF1;
+  const __amdgpu_buffer_rsrc_t xb = msfec_wave::buffer_of(out, 3 * C::NF1 * 8);
+  const int face[3] = {((k0 * M + j) * S + i) * 8, (C::NF1 + (k0 * S + j) * M + i) * 8,
+                       (2 * C::NF1 + (k0 * M + j) * M + i) * 8};
+  auto step = [](int d) { return (d == 2 ? M2 : M * S) * 8; };  // to the next cell of the column
   // q = M_A p on the lower faces: x and z parts in the lattice (z of the first
   // cell, whose place the segment below reads, in qz), y part in qy without
   // what U brings, z of the first cell without what V brings; returns
@@ -323,11 +332,11 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
     const int lev[3] = {i, j, k0 + t};
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      const int step = d == 0 ? 1 : (d == 1 ? S : S * S);
+      const int next = d == 0 ? 1 : (d == 1 ? S : S * S);
       const double* e = E + d * S3 + at0 + t * S * S;
-      x[d][t] = 0.0;
+      if (on) buffer_f64(xb, face[d], t * step(d), 0.0);
       p[d][t] = e[0];
-      r[d][t] = lev[d] > 0 ? mf[d] * fma(2.0 / 3.0, e[0], (e[-step] + e[step]) * (1.0 / 6.0)) : 0.0;
+      r[d][t] = lev[d] > 0 ? mf[d] * fma(2.0 / 3.0, e[0], (e[-next] + e[next]) * (1.0 / 6.0)) : 0.0;
     }
   }
   const double stop = g.rtol * g.rtol * rz;
@@ -352,13 +361,20 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
       break;
     }
     const double alpha = rz / pq;
+    double x[2][3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) x[0][d] = buffer_f64(xb, face[d], 0);
 #pragma unroll
     for (int t = 0; t < LZ; ++t) {
+      if (t + 1 < LZ)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) x[(t + 1) & 1][d] = buffer_f64(xb, face[d], (t + 1) * step(d));
+      __builtin_amdgcn_sched_barrier(0);
       double q[3];
       product(t, q);
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        x[d][t] = fma(alpha, p[d][t], x[d][t]);
+        if (on) buffer_f64(xb, face[d], t * step(d), fma(alpha, p[d][t], x[t & 1][d]));
         r[d][t] = fma(-alpha, q[d], r[d][t]);
         if (on) E[d * S3 + at0 + t * S * S] = r[d][t];
       }
@@ -374,14 +390,15 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
     ++it;
   }
   if (!isfinite(rz)) flag = MSFEC_CELL_NONFINITE;
-  double* out = g.S + ((size_t)cell * 6 + nb) * 3 * C::NF1;
 #pragma unroll
   for (int t = 0; t < LZ; ++t) {
     if (!on) break;
-    const int k = k0 + t;
-    out[(k * M + j) * S + i] = coarse(0, i) + (i > 0 ? x[0][t] : 0.0);
-    out[C::NF1 + (k * S + j) * M + i] = coarse(1, j) + (j > 0 ? x[1][t] : 0.0);
-    out[2 * C::NF1 + (k * M + j) * M + i] = coarse(2, k) + (k > 0 ? x[2][t] : 0.0);
+    const int k = k0 + t, lev[3] = {i, j, k};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const double x = buffer_f64(xb, face[d], t * step(d));
+      buffer_f64(xb, face[d], t * step(d), coarse(d, lev[d]) + (lev[d] > 0 ? x : 0.0));
+    }
     if (i == M - 1) out[(k * M + j) * S + M] = coarse(0, M);
     if (j == M - 1) out[C::NF1 + (k * S + M) * M + i] = coarse(1, M);
     if (k == M - 1) out[2 * C::NF1 + (M * M + j) * M + i] = coarse(2, M);

@@ -17,6 +17,10 @@ __device__ __forceinline__ double buffer_f64(__amdgpu_buffer_rsrc_t b, int lane,
   const buffer_v2 t = __builtin_amdgcn_raw_buffer_load_b64(b, lane, uni, 0);
   return __hiloint2double((int)t.y, (int)t.x);
 }
+__device__ __forceinline__ void buffer_f64(__amdgpu_buffer_rsrc_t b, int lane, int uni, double v) {
+  const buffer_v2 t = {(unsigned)__double2loint(v), (unsigned)__double2hiint(v)};
+  __builtin_amdgcn_raw_buffer_store_b64(t, b, lane, uni, 0);
+}
 
 // Sum over the N lanes (a power of two, at most 16) of a row, or of N values
 // that repeat within it: every lane has it, in the same bits, as a + b = b + a.
