@@ -7,8 +7,15 @@
 
 namespace msfec_detail {
 
-// 2^l fine cells per direction, 2^l - 1 inner nodes.  Whether there is a kernel.
-inline bool lines_has(int l) { return l == 4 || l == 5; }
+// 2^l fine cells per direction, 2^l - 1 inner nodes.  Whether there is a kernel
+// and it is the faster one: below l = 4 a line is less than a tile, and many
+// cells fill the card with the band factorisation's one wave each, which takes
+// fewer operations.  A pass of 2-D RT_DQ, band and this: l = 4 1 cell 108 and 50
+// us, 1024 159 and 125, 2025 236 and 238, 4096 473 and 493; l = 5 1 cell 497 and
+// 172, 400 569 and 399, 625 619 and 593, 784 667 and 779.
+inline bool lines_has(int l, int n_cells) {
+  return (l == 4 && n_cells <= 1536) || (l == 5 && n_cells <= 640);
+}
 // Scratch per cell in doubles.
 size_t lines_doubles(int l);
 // K X = R for a batch of symmetric positive definite systems.  rows

@@ -31,12 +31,12 @@
 //                      the 4 right-hand sides, from exact integrals with 1/a
 //                      staged in LDS, or, for a tensor A given at the
 //                      QGauss(2) points, by that rule with A^-1 at each point.
-//   lines_solve        (msfec_lines.hip) for l = 4 and 5: block cyclic
-//                      reduction over the lines of nodes.
+//   lines_solve        (msfec_lines.hip) for l = 4 and 5 and not too many
+//                      cells: block cyclic reduction over the lines of nodes.
 //   band_ldl_solve     (msfec_q.hip) one wave per cell: the matrix-core band
 //                      L D L^T, 4 pivots per step, with the forward
-//                      elimination and the backward sweep; for l < 4 and the
-//                      cells that are not positive definite.
+//                      elimination and the backward sweep; otherwise, and for
+//                      the cells that are not positive definite.
 //   rt_element_kernel  one workgroup per cell: psi in LDS, the fine fluxes of
 //                      the 4 bases to HBM and the 5 x 5 element matrix and
 //                      load from exact integrals per fine cell (QGauss(2)
@@ -592,7 +592,7 @@ msfec_status msfec_rt_create(const msfec_rt_params* params, int n_cells, const d
   RT_TRY(rt_alloc(&h->d_f, nc * nf));
   RT_TRY(rt_alloc(&h->d_rows, nc * h->n * kRowLen));
   RT_TRY(rt_alloc(&h->d_pan, nc * std::max(msfec_detail::band_ldl_panel_doubles(h->n),
-                                           msfec_detail::lines_has(l) ? msfec_detail::lines_doubles(l) : 0)));
+                                           msfec_detail::lines_has(l, n_cells) ? msfec_detail::lines_doubles(l) : 0)));
   RT_TRY(rt_alloc(&h->d_zst, nc * msfec_detail::band_ldl_z_doubles(h->n)));
   RT_TRY(rt_alloc(&h->d_X, nc * h->n * kNR));
   RT_TRY(rt_alloc(&h->d_sigma, nc * kNB * h->ne));
@@ -657,11 +657,10 @@ msfec_status msfec_rt_compute(msfec_rt_handle h, void* stream) {
     RT_HIP(hipGetLastError());
   }
   if (ev) RT_HIP(hipEventRecord((*ev)[1], s));
-  // by lines where there is a kernel (1024 cells at l = 4 71 us, 111 by the band
-  // solve; 121 at l = 5 145 and 463; below, a line is less than a tile), and
-  // then the band L D L^T, which takes pivots of either sign, for the cells that
-  // are not positive definite (4.5 us where there are none)
-  const bool lines = msfec_detail::lines_has(h->prm.n_refine_local);
+  // by lines where that is faster, and then the band L D L^T, which takes pivots
+  // of either sign, for the cells that are not positive definite (4.5 us where
+  // there are none)
+  const bool lines = msfec_detail::lines_has(h->prm.n_refine_local, h->n_cells);
   if (lines)
     RT_HIP(msfec_detail::lines_solve(h->prm.n_refine_local, h->n_cells, h->d_rows, h->d_pan, h->d_X,
                                      h->d_status, s));

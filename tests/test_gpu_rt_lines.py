@@ -55,3 +55,18 @@ def test_not_positive_definite(l, tensor):
     assert np.abs(S[1] - S[0]).max() <= TOL_S * np.abs(S[0]).max()
     assert np.abs(M[1, :4, :4] + M[0, :4, :4]).max() <= TOL_M * np.abs(M[0, :4, :4]).max()
     assert np.array_equal(S[3], S[0]) and np.isfinite(S[4]).all()
+
+
+@pytest.mark.parametrize("l,n", [(4, 1536), (4, 1537), (5, 640), (5, 641)])
+def test_sides_of_the_rule(l, n):
+    """The same cells by lines and, one cell more, by the band solve."""
+    print(f"case rt lines rule l={l} n={n}", flush=True)
+    rng = np.random.default_rng(970 + l)
+    verts, a = boxes(rng, 4), coefficient(rng, 4, l, False)
+    pick = np.arange(n) % 4
+    M, _, S, st = run_gpu(verts[pick], l, a[pick], 1.0)
+    few, _, Sf, _ = run_gpu(verts, l, a, 1.0)
+    assert (st == 0).all()
+    for c in (0, 1, 2, 3, n - 1):
+        assert np.abs(S[c] - Sf[c % 4]).max() <= TOL_S * np.abs(Sf[c % 4]).max()
+        assert np.abs(M[c, :4, :4] - few[c % 4, :4, :4]).max() <= TOL_M * np.abs(few[c % 4, :4, :4]).max()
