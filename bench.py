@@ -325,13 +325,14 @@ def rt_config(steps: int, warmup: int, check: bool, cpu: bool):
     out = {"workload": "2D Raviart-Thomas x DQ0 basis, 32x32=1024 coarse cells x 16x16 fine "
                        "cells (544 fluxes + 256 cell values per basis, 4 face bases); the flux "
                        "is the coarse function plus the curl of a Q1 stream function: 225 "
-                       "unknowns, half-bandwidth 16, band LDL^T FP64 on the matrix cores",
+                       "unknowns, block cyclic reduction over the lines of nodes, FP64 on the "
+                       "matrix cores (flops: those of a band LDL^T of half-bandwidth 16)",
            "cells_per_s": round(n_cells / (wall / steps), 1),
            "ms_per_step": round(wall * 1e3 / steps, 4),
            "kernel_ms": {"rows": round(kt[0], 4), "factor_solve": round(kt[1], 4),
                          "flux_element": round(kt[2], 4)},
            "failed_cells": int((rb.get_cell_status() != 0).sum()),
-           "roofline": {"bound": "mfma", "kernel": "q_blk_factor_kernel<double, 2, 1, true>",
+           "roofline": {"bound": "mfma", "kernel": "lines_kernel<1>",
                         "flops_per_cell": flops_cell, "achieved_tflops": round(tflops, 4),
                         "peak_tflops": FP64_PEAK_TFLOPS,
                         "frac": round(tflops / FP64_PEAK_TFLOPS, 5)},
@@ -368,13 +369,6 @@ def rt_config(steps: int, warmup: int, check: bool, cpu: bool):
 NRT_NREF, NRT_NC = 2, 16
 
 
-def nrt_flops_per_cell(n: int, nrhs: int) -> float:
-    """Algorithmic FP64 flops of the dense symmetric indefinite L D L^T of an
-    n x n system (n^3 / 3) and its forward and backward sweeps for nrhs
-    right-hand sides (2 n^2 each)."""
-    return n ** 3 / 3.0 + 2.0 * n * n * nrhs
-
-
 def nrt_config(steps: int, warmup: int, check: bool, cpu: bool):
     """The 3-D Nedelec x Raviart-Thomas configuration: 16^3 coarse cells of the
     unit cube, 4^3 fine cells each (300 edges + 240 faces; 108 + 144 = 252
@@ -403,28 +397,23 @@ def nrt_config(steps: int, warmup: int, check: bool, cpu: bool):
     wall = time.perf_counter() - t0
     kt = nb.kernel_times()
     m = 1 << NRT_NREF
-    n_int = 3 * m * (m - 1) ** 2 + 3 * (m - 1) * m * m
-    flops_cell = nrt_flops_per_cell(n_int, 18)
-    tflops = flops_cell * n_cells / (kt[0] * 1e-3) / 1e12
     # compulsory HBM bytes per cell: the Gauss-point coefficients in (6 + 1 + 3
     # values at 8 points of 64 fine cells), the 18 fine vectors, M and b out
     hbm_cell = 8.0 * (m ** 3 * 8 * 10 + 18 * nb.N + 18 * 18 + 18)
     out = {"workload": "3D Nedelec x Raviart-Thomas basis, 16^3=4096 coarse cells x 4^3 fine "
                        "cells (300 edges + 240 faces, 252 interior unknowns), 12 edge + 6 face "
-                       "bases, coefficients of prm_ned_rt_test-01 at the Gauss points; one "
-                       "workgroup per cell: dense symmetric indefinite L D L^T FP64 on the "
-                       "matrix cores with the 18 right-hand sides, backward sweep, element matrix",
+                       "bases, coefficients of prm_ned_rt_test-01 at the Gauss points; "
+                       "by the discrete exact sequence (scalar Q1 potentials, Gauss-Jordan)",
            "cells_per_s": round(n_cells / (wall / steps), 1),
            "ms_per_step": round(wall * 1e3 / steps, 4),
            "kernel_ms": {"basis": round(kt[0], 4)},
            "failed_cells": int((nb.get_cell_status() != 0).sum()),
-           "roofline": {"bound": "mfma", "kernel": "nrt_basis_kernel<2>",
-                        "flops_per_cell": flops_cell, "achieved_tflops": round(tflops, 4),
-                        "peak_tflops": FP64_PEAK_TFLOPS,
-                        "frac": round(tflops / FP64_PEAK_TFLOPS, 5),
-                        "hbm_bytes_per_cell": hbm_cell,
-                        "hbm_frac": round(hbm_cell * n_cells / (kt[0] * 1e-3) / 1e9
-                                          / HBM_PEAK_GBS, 5)}}
+           "roofline": {"bound": "hbm", "kernel": "all kernels of a step",
+                        "bytes_per_cell": hbm_cell,
+                        "achieved_gbs": round(hbm_cell * n_cells / (kt[0] * 1e-3) / 1e9, 1),
+                        "peak_gbs": HBM_PEAK_GBS,
+                        "frac": round(hbm_cell * n_cells / (kt[0] * 1e-3) / 1e9
+                                      / HBM_PEAK_GBS, 5)}}
     if check or cpu:
         from oracle import oracle as O
         O.build()
@@ -457,30 +446,12 @@ def nrt_config(steps: int, warmup: int, check: bool, cpu: bool):
 NRT4_NREF, NRT4_NC = 4, 4
 
 
-def nrt_minres_bytes_per_iteration(n: int, ns: int, nu: int, nfc: int, nc0: int,
-                                   edge_schwarz: bool) -> float:
-    """Algorithmic bytes of one MINRES iteration of one basis: 16 passes over
-    the n interior values (the product reads v once and reads and writes the
-    first residual slot; the second pass reads both residuals and the
-    preconditioner and writes one; the third reads v, w, w2, x, the new
-    residual and the preconditioner and writes w, x and v); a share of the
-    cell's local matrices (99 values per fine cell, read by the 18 bases);
-    the coarse correction (the nu face values restricted, the nc0 x nc0
-    inverse read); and, with the edge additive Schwarz, 5 passes over the ns
-    interior edges (z cleared, y gathered, z read and written, z read for
-    the next v) and a share of the 78 inverse entries per fine cell."""
-    b = 16 * n + 99 * nfc / 18.0 + nu + nc0 * nc0
-    if edge_schwarz:
-        b += 5 * ns + 78 * nfc / 18.0
-    return 8.0 * b
-
-
 def nrt4_config(steps: int, warmup: int, check: bool, cpu: bool):
     """The reference's own Ned_RT example: prm_ned_rt_test-01 (global
     refinements 2: 4^3 = 64 coarse cells of the unit cube; local refinements
     4: 16^3 fine cells per coarse cell, 13 872 edges + 13 056 faces, 22 320
     interior unknowns), its coefficients at the Gauss points, 12 edge + 6
-    face bases, solved by matrix-free MINRES."""
+    face bases, by the discrete exact sequence and CG on scalar Q1 potentials."""
     from msfec_amd import NedRTBasisBatch, fields as F
     verts = F.box_grid_3d(NRT4_NC)
     pts = F.gauss_points_3d(verts, NRT4_NREF)
@@ -503,26 +474,23 @@ def nrt4_config(steps: int, warmup: int, check: bool, cpu: bool):
     kt = nb.kernel_times()
     its = nb.get_iterations()
     m = 1 << NRT4_NREF
-    ns, nu = 3 * m * (m - 1) ** 2, 3 * (m - 1) * m * m
-    nblk = m // 2 if m <= 4 else 4  # aggregates per direction of the coarse correction
-    bpi = nrt_minres_bytes_per_iteration(ns + nu, ns, nu, m ** 3, 3 * nblk ** 3, NRT4_NREF >= 4)
-    gbs = float(its.sum()) * bpi / (kt[2] * 1e-3) / 1e9
+    # compulsory HBM bytes: the Gauss-point coefficients in, the bases, M and b out
+    hbm_cell = 8.0 * (m ** 3 * 8 * 10 + 18 * nb.N + 18 * 18 + 18)
+    gbs = hbm_cell * n_cells / (kt[0] * 1e-3) / 1e9
     out = {"workload": "3D Nedelec x Raviart-Thomas basis, the reference's prm_ned_rt_test-01: "
                        "4^3=64 coarse cells x 16^3 fine cells (13872 edges + 13056 faces, "
                        "22320 interior unknowns), 12 edge + 6 face bases, its coefficients at "
-                       "the Gauss points; matrix-free MINRES (relative tolerance 1e-14) "
-                       "preconditioned by an element additive Schwarz on the edges and a "
-                       "diagonal plus 192-dof coarse correction on the faces, one workgroup "
-                       "per basis",
+                       "the Gauss points; by the discrete exact sequence, CG on scalar Q1 "
+                       "potentials",
            "cells_per_s": round(n_cells / (wall / steps), 2),
            "ms_per_step": round(wall * 1e3 / steps, 3),
-           "kernel_ms": {"total": round(kt[0], 3), "local_and_preconditioner": round(kt[1], 3),
-                         "minres": round(kt[2], 3), "element": round(kt[3], 3)},
-           "minres_iterations": {"mean": round(float(its.mean()), 1), "min": int(its.min()),
+           "kernel_ms": {"total": round(kt[0], 3), "fluxes_and_rows": round(kt[1], 3),
+                         "solve": round(kt[2], 3), "element": round(kt[3], 3)},
+           "cg_iterations": {"mean": round(float(its.mean()), 1), "min": int(its.min()),
                                  "max": int(its.max())},
            "failed_cells": int((nb.get_cell_status() != 0).sum()),
-           "roofline": {"bound": "hbm", "kernel": "nrt_minres_kernel<4>",
-                        "bytes_per_iteration_basis": bpi, "achieved_gbs": round(gbs, 1),
+           "roofline": {"bound": "hbm", "kernel": "all kernels of a step",
+                        "bytes_per_cell": hbm_cell, "achieved_gbs": round(gbs, 1),
                         "peak_gbs": HBM_PEAK_GBS, "frac": round(gbs / HBM_PEAK_GBS, 4)}}
     if check or cpu:
         from oracle import oracle as O
@@ -552,16 +520,6 @@ def nrt4_config(steps: int, warmup: int, check: bool, cpu: bool):
 RT3_NREF, RT3_NC = 4, 4
 
 
-def rt3_cg_bytes_per_iteration(nfc: int, ns: int) -> float:
-    """Algorithmic HBM bytes of one Jacobi-PCG iteration of one 3-D RT_DQ
-    basis (vectors over the ns interior edges): the 21 face-mass entries of
-    every fine cell, p read and q read and written in the element-by-element
-    product, then per edge x and r read and written, p, q and the Jacobi
-    diagonal read in the update (56 B), and the diagonal, r, p read, p and q
-    written in the direction update (40 B)."""
-    return 8.0 * 21 * nfc + 24.0 * ns + 96.0 * ns
-
-
 def rt3_config(steps: int, warmup: int, check: bool, cpu: bool):
     """The reference's own 3-D RT_DQ example, prm_rt_dq_test-01 (global
     refinements 2: 4^3 = 64 coarse cells of the unit cube; local refinements
@@ -588,15 +546,14 @@ def rt3_config(steps: int, warmup: int, check: bool, cpu: bool):
     kt = rb.kernel_times()
     its = rb.get_iterations()
     m = 1 << RT3_NREF
-    ns = 3 * m * (m - 1) ** 2
-    bpi = rt3_cg_bytes_per_iteration(m ** 3, ns)
-    gbs = float(its.sum()) * bpi / (kt[2] * 1e-3) / 1e9
+    # compulsory HBM bytes: A^-1 and f at the Gauss points in, the fluxes, M and b out
+    hbm_cell = 8.0 * (m ** 3 * 8 * 7 + 6 * 3 * m * m * (m + 1) + 56)
+    gbs = hbm_cell * n_cells / (kt[0] * 1e-3) / 1e9
     out = {"workload": "3D Raviart-Thomas x DQ0 basis, the reference's prm_rt_dq_test-01: "
                        "4^3=64 coarse cells x 16^3 fine cells (13056 faces + 4096 cell values), "
                        "6 face bases, its coefficients and right-hand side at the Gauss points; "
-                       "the flux is the coarse function plus the curl of an interior Nedelec "
-                       f"field ({ns} interior edges), curl-curl system by Jacobi-PCG "
-                       "(relative tolerance 1e-13), one workgroup per basis",
+                       "CG on the fluxes, projected onto the divergence-free ones, one "
+                       "workgroup per basis",
            "cells_per_s": round(n_cells / (wall / steps), 2),
            "ms_per_step": round(wall * 1e3 / steps, 3),
            "kernel_ms": {"total": round(kt[0], 3), "local_and_diagonal": round(kt[1], 3),
@@ -604,8 +561,8 @@ def rt3_config(steps: int, warmup: int, check: bool, cpu: bool):
            "cg_iterations": {"mean": round(float(its.mean()), 1), "min": int(its.min()),
                              "max": int(its.max())},
            "failed_cells": int((rb.get_cell_status() != 0).sum()),
-           "roofline": {"bound": "hbm", "kernel": "rt3_cg_kernel<4>",
-                        "bytes_per_iteration_basis": bpi, "achieved_gbs": round(gbs, 1),
+           "roofline": {"bound": "hbm", "kernel": "all kernels of a step",
+                        "bytes_per_cell": hbm_cell, "achieved_gbs": round(gbs, 1),
                         "peak_gbs": HBM_PEAK_GBS, "frac": round(gbs / HBM_PEAK_GBS, 4)}}
     if check or cpu:
         from oracle import oracle as O
