@@ -308,6 +308,7 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
     transform<M, NT, ModesToFace>(E, 3);
     return waves_sum<C::NW>(red + C::NW);
   };
+  __syncthreads();  // the lattice is zeroed: its points belong to other threads below
   apply(true);
   __syncthreads();
 #pragma unroll

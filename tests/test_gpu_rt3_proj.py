@@ -69,3 +69,25 @@ def test_general_cells_do_not_disturb_others(l):
         assert got[3][c] == 0
         for k in range(3):
             np.testing.assert_array_equal(got[k][c], good[k][c])
+
+
+@pytest.mark.parametrize("l,n", [(3, 300), (4, 50)])
+def test_equal_cells_come_out_equal(l, n):
+    """More workgroups than the card runs at once, all with the same data, over
+    several passes: every cell bit for bit the same (the waves of a workgroup
+    share their flux lattice, so the order in which they run must not show)."""
+    print(f"case rt3 equal cells l={l} n={n}", flush=True)
+    from msfec_amd import RTDQ3BasisBatch
+    rng = np.random.default_rng(5200 + l)
+    verts = np.repeat(boxes(rng, 1), n, 0)
+    ainv, _, _, _ = rand_coefs(rng, 1, l, reaction=False, load=False)
+    one = run(verts[:1], l, ainv)
+    assert one[3][0] == 0
+    with RTDQ3BasisBatch(verts, n_refine_local=l) as rb:
+        rb.set_coefficients(np.repeat(ainv, n, 0))
+        for _ in range(3):
+            rb.run()
+            got = (rb.get_global_element_matrix(), rb.get_global_element_rhs(), rb.get_basis(),
+                   rb.get_cell_status(), rb.get_iterations())
+            for a, b in zip(got, one):
+                np.testing.assert_array_equal(a, np.broadcast_to(b, a.shape))
