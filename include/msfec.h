@@ -239,7 +239,9 @@ void msfec_q_destroy(msfec_q_handle h);
  * by Jacobi-preconditioned CG in FP64 on the device until
  * ||r|| <= max(abs_tol, rel_tol ||b||).  u (n_nodes doubles, loc) receives the
  * nodal solution, zero on the boundary; iterations and the final residual are
- * returned.  Replaces QMultiscale::assemble_system, solve_iterative and the
+ * returned.  MSFEC_ERR_CELL, with minus the iterations, where max_iter is
+ * reached, the matrix turns out not to be positive definite, or the residual
+ * is not finite.  Replaces QMultiscale::assemble_system, solve_iterative and the
  * weight extraction of send_global_weights_to_cell
  * (source/Q/q_global.cc:198-297, 327-363, 368-392). */
 msfec_status msfec_coarse_solve(msfec_q_handle h, int nc, double abs_tol,

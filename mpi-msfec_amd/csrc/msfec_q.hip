@@ -3009,6 +3009,13 @@ __device__ double block_sum(double v, double* red) {
   return s;
 }
 
+// What a coarse solve reports: its iterations, or -1 - iterations where the
+// residual did not come down to the bound (the limit, a matrix that is not
+// positive definite) or is not finite.
+__device__ __forceinline__ int coarse_iterations(int it, double rr, double stop) {
+  return (rr <= stop && isfinite(rr)) ? it : -1 - it;
+}
+
 __global__ __launch_bounds__(1024) void coarse_cg_kernel(int dim, int nc, const double* __restrict__ K,
                                                          const double* __restrict__ rhs,
                                                          double* __restrict__ u, double* r,
@@ -3081,7 +3088,7 @@ __global__ __launch_bounds__(1024) void coarse_cg_kernel(int dim, int nc, const 
     ++it;
   }
   if (threadIdx.x == 0) {
-    *iters_out = (rnorm2 > stop) ? -it : it;
+    *iters_out = coarse_iterations(it, rnorm2, stop);
     *res_out = sqrt(rnorm2);
   }
 }
@@ -3205,7 +3212,7 @@ __global__ __launch_bounds__(kCoarseThreads) void coarse_pcg_kernel(
     ++it;
   }
   if (tid == 0) {
-    *iters_out = (rr > stop) ? -it : it;
+    *iters_out = coarse_iterations(it, rr, stop);
     *res_out = sqrt(rr);
   }
 }
@@ -3323,7 +3330,7 @@ __global__ __launch_bounds__(kCoarseThreads) void coarse_pcg_reg_kernel(
   for (int t = 0; t < T; ++t)
     if (tid + t * nt < nint) u[id[t]] = x[t];
   if (tid == 0) {
-    *iters_out = (rr > stop) ? -it : it;
+    *iters_out = coarse_iterations(it, rr, stop);
     *res_out = sqrt(rr);
   }
 }
@@ -4256,7 +4263,8 @@ hipError_t band_ldl_mixed_solve(int n_cells, int n, int bw, const double* rows, 
 // element data of the nc^dim structured coarse grid (cells lexicographic):
 // dM [cells][2^dim][2^dim], db [cells][2^dim].  Buffers: cK [3^dim][nodes],
 // crhs [nodes], cvec [5 nodes + 1 + cells 2^dim] (u | r | z | p | q |
-// final residual | weights), cit [1].  Enqueued on s.
+// final residual | weights), cit [1] (iterations, or -1 - iterations for a
+// solve that failed).  Enqueued on s.
 hipError_t coarse_solve_device(int dim, int nc, const double* dM, const double* db, double* cK,
                                double* crhs, double* cvec, int* cit, double abs_tol,
                                double rel_tol, int max_iter, hipStream_t s) {
@@ -5163,7 +5171,7 @@ msfec_status msfec_coarse_solve(msfec_q_handle h, int nc, double abs_tol, double
   MSFEC_HIP(hipMemcpyAsync(&it, h->d_cit, sizeof(int), hipMemcpyDeviceToHost, h->stream));
   MSFEC_HIP(hipMemcpyAsync(&rr, res, sizeof(double), hipMemcpyDeviceToHost, h->stream));
   MSFEC_HIP(hipStreamSynchronize(h->stream));
-  if (iterations) *iterations = it;
+  if (iterations) *iterations = it < 0 ? it + 1 : it;
   if (residual) *residual = rr;
   if (it < 0) return fail(MSFEC_ERR_CELL, "coarse CG did not converge");
   return MSFEC_OK;

@@ -593,7 +593,7 @@ msfec_status msfec_qu_coarse_solve(msfec_qu_handle h, int nc, double abs_tol, do
   const double* dw = res + 1;
   QU_HIP(hipMemcpy(&it, h->d_cit, sizeof(int), hipMemcpyDeviceToHost));
   QU_HIP(hipMemcpy(&rr, res, sizeof(double), hipMemcpyDeviceToHost));
-  if (iterations) *iterations = it;
+  if (iterations) *iterations = it < 0 ? it + 1 : it;
   if (residual) *residual = rr;
   auto out = [&](double* dst, const double* src, size_t count, int loc) -> msfec_status {
     QU_HIP(hipMemcpyAsync(dst, src, count * sizeof(double),

@@ -40,3 +40,65 @@ def test_coarse_residual(dim, nc):
     true = np.linalg.norm((rhs - K @ u)[free])
     assert true <= 1e-12 * np.linalg.norm(rhs[free]) + gap, (true, res, gap)
     assert res <= 1e-12 * np.linalg.norm(rhs[free])
+
+
+@pytest.mark.parametrize("dim,nc", [(2, 9), (2, 34), (2, 66), (2, 115), (3, 5), (3, 12), (3, 18)])
+def test_coarse_failures(dim, nc):
+    """A load that is not finite, a matrix that is not (the solve fails before
+    its first iteration) or that is negative definite (at its first step), and
+    a limit of no iterations are errors on every kernel, and leave the handle
+    fit for the next solve."""
+    print(f"case coarse failures dim={dim} nc={nc}", flush=True)
+    from msfec_amd import QBasisBatch, _lib as L
+    from msfec_amd import fields as F
+    n, nf = nc ** dim, 1 << dim
+    coef, f = np.ones((n, nf)), np.ones((n, nf))
+    with QBasisBatch(F.coarse_vertices(dim, nc), dim=dim, n_refine_local=1,
+                     rhs_mode=L.RHS_CELL) as qb:
+        def fails(c, load, **kw):
+            qb.set_coefficient(c)
+            qb.set_rhs(load)
+            qb.run()
+            with pytest.raises(RuntimeError, match="did not converge"):
+                qb.coarse_solve(nc, abs_tol=0.0, rel_tol=1e-12, **kw)
+
+        for v in (np.nan, np.inf, -np.inf):
+            g = f.copy()
+            g[n // 2, 0] = v
+            fails(coef, g)
+        c = coef.copy()
+        c[n // 2, 0] = np.nan
+        fails(c, f)
+        if nc < 100:  # the general kernel takes a negative definite matrix
+            fails(-coef, f)
+        fails(coef, f, max_iter=0)
+        qb.set_coefficient(coef)
+        qb.set_rhs(0 * f)
+        qb.run()
+        u, _, it, res = qb.coarse_solve(nc, abs_tol=0.0, rel_tol=1e-12)
+        assert it == 0 and res == 0.0 and (u == 0.0).all()
+        qb.set_rhs(f)
+        qb.run()
+        u, _, it, res = qb.coarse_solve(nc, abs_tol=0.0, rel_tol=1e-12)
+        assert it > 0 and u.max() > 0.0
+
+
+def test_adjoint_failures():
+    """The gradient goes by the same solves: a target that is not finite is an
+    error inside and does not count on the boundary."""
+    print("case adjoint failures", flush=True)
+    from msfec_amd import QBasisBatch, _lib as L
+    from msfec_amd import fields as F
+    nc = 4
+    with QBasisBatch(F.coarse_vertices(3, nc), dim=3, n_refine_local=1,
+                     solver=L.SOLVER_BAND_FP64_MFMA) as qb:
+        qb.set_coefficient(np.ones((nc ** 3, 8)))
+        qb.run()
+        t = np.zeros((nc + 1,) * 3)
+        J, g = qb.adjoint_gradient(nc, t)
+        t[0] = np.nan
+        Jb, gb = qb.adjoint_gradient(nc, t)
+        assert Jb == J and np.array_equal(gb, g)
+        t[2, 2, 2] = np.nan
+        with pytest.raises(RuntimeError, match="did not converge"):
+            qb.adjoint_gradient(nc, t)
