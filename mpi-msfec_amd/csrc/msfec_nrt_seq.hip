@@ -79,6 +79,7 @@ __global__ __launch_bounds__(1024) void nrt_seq_weights_kernel(NrtSeq g) {
       s += t.x;
       s += t.y;
     }
+    bad |= !isfinite(s);  // an infinite B would only lower the weight to 0
     const double w = vol / (s * 0.125);
     W[c] = w;
     sum += w;

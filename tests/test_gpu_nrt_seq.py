@@ -98,3 +98,27 @@ def test_iteration_limit():
     ainv, bq, _, fq = rand_coefs(rng, 2, 3, reaction=False)
     _, _, _, st, its = run(verts, 3, ainv, bq, None, fq, max_iter=5)
     assert (st == L.CELL_NOT_CONVERGED).all() and (its[:, :12] == 5).all()
+
+
+@pytest.mark.parametrize("l", [1, 2, 3])
+def test_infinite_data(l):
+    """An infinite B or A^-1 at one Gauss point, and values of B whose sum over
+    a fine cell overflows: flagged, never MSFEC_CELL_OK; a large
+    finite value of B passes."""
+    print(f"case nrt sequence infinite data l={l}", flush=True)
+    rng = np.random.default_rng(3400 + l)
+    n = 7
+    verts = boxes(rng, n)
+    ainv, bq, _, fq = rand_coefs(rng, n, l, reaction=False)
+    good = run(verts, l, ainv, bq, None, fq, max_iter=400)
+    bq[1, 0, 3] = np.inf
+    bq[2, -1, 7] = np.inf
+    bq[3, 1, :] = 1e308
+    ainv[4, 2, 5, 3] = np.inf
+    bq[5, 0, 0] = 1e307
+    a = run(verts, l, ainv, bq, None, fq, max_iter=400)
+    assert (a[3][[1, 2, 3, 4]] != 0).all(), a[3]
+    assert (a[3][[0, 5, 6]] == 0).all(), a[3]
+    for c in (0, 6):
+        for k in range(3):
+            np.testing.assert_array_equal(a[k][c], good[k][c])
