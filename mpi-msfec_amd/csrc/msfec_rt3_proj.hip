@@ -174,7 +174,12 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
   const int col = own % M2, seg = own / M2, i = col % M, j = col / M, k0 = seg * LZ;
   double H[3], h[3];
   sizes(g.verts + (size_t)cell * 24, M, H, h);
-  const double mf[3] = {h[0] / (h[1] * h[2]), h[1] / (h[0] * h[2]), h[2] / (h[0] * h[1])};
+  // the mass of the projection in units of A^-1 (a power of two: no rounding), so that
+  // p is of the size of the flux and p . M_A p linear in A^-1; with the plain mass it is
+  // cubic and falls below the range of a double for A^-1 = 1e-100
+  const double unit = ldexp(1.0, ilogb(top));
+  const double mf[3] = {unit * (h[0] / (h[1] * h[2])), unit * (h[1] / (h[0] * h[2])),
+                        unit * (h[2] / (h[0] * h[1]))};
   for (int e = tid; e < 3 * S3; e += NT) E[e] = 0.0;
   if (tid < M) {
     kap[tid] = 2.0 * sinpi(tid * (0.5 / M));

@@ -91,3 +91,24 @@ def test_equal_cells_come_out_equal(l, n):
                    rb.get_cell_status(), rb.get_iterations())
             for a, b in zip(got, one):
                 np.testing.assert_array_equal(a, np.broadcast_to(b, a.shape))
+
+
+@pytest.mark.parametrize("l", [1, 2, 3, 4])
+def test_units_of_the_coefficient(l):
+    """A^-1 in other units, from 2^-320 to 2^330 (about 1e-96 and 1e99): the
+    same fluxes and iterations bit for bit, the flux block of M scaled."""
+    print(f"case rt3 units l={l}", flush=True)
+    rng = np.random.default_rng(5300 + l)
+    n = 3
+    verts = boxes(rng, n)
+    ainv = np.zeros((n, 8 ** l, 8, 6))
+    ainv[..., [0, 3, 5]] = np.exp(0.5 * rng.normal(size=(n, 8 ** l, 8, 3)))
+    ainv[..., 1] = 0.1 * ainv[..., 0]
+    want = run(verts, l, ainv)
+    assert (want[3] == 0).all()
+    for e in (-320, -100, 100, 330):
+        got = run(verts, l, ainv * 2.0 ** e, max_iter=1000)
+        assert (got[3] == 0).all(), (e, got[3], got[4].max())
+        np.testing.assert_array_equal(got[2], want[2])
+        np.testing.assert_array_equal(got[4], want[4])
+        np.testing.assert_array_equal(got[0][:, :6, :6], want[0][:, :6, :6] * 2.0 ** e)
