@@ -112,3 +112,25 @@ def test_units_of_the_coefficient(l):
         np.testing.assert_array_equal(got[2], want[2])
         np.testing.assert_array_equal(got[4], want[4])
         np.testing.assert_array_equal(got[0][:, :6, :6], want[0][:, :6, :6] * 2.0 ** e)
+
+
+@pytest.mark.parametrize("l", [1, 2, 3, 4])
+@pytest.mark.parametrize("dev", [0.3, 1.0, 1.5, 2.0])
+def test_balance_of_every_fine_cell(l, dev):
+    """The net outflow of a fine cell is -+1/M^3, to the rounding of its 6
+    fluxes and of their sum here (each at most half a unit in the last place
+    of the largest flux): 6 eps of it, whatever the iterations."""
+    print(f"case rt3 balance l={l} deviation={dev}", flush=True)
+    rng = np.random.default_rng(5400 + l)
+    n, m = 4, 1 << l
+    ainv = np.zeros((n, m ** 3, 8, 6))
+    ainv[..., [0, 3, 5]] = np.exp(dev * rng.normal(size=(n, m ** 3, 1, 1)))
+    _, _, S, st, _ = run(boxes(rng, n), l, ainv)
+    assert (st == 0).all()
+    x, y, z = np.split(S, 3, -1)
+    x = np.diff(x.reshape(n, 6, m, m, m + 1), axis=4)
+    y = np.diff(y.reshape(n, 6, m, m + 1, m), axis=3)
+    z = np.diff(z.reshape(n, 6, m + 1, m, m), axis=2)
+    want = np.array([-1.0, 1, -1, 1, -1, 1])[None, :, None, None, None] / m ** 3
+    off = np.abs(x + y + z - want).max((2, 3, 4)) / np.abs(S).max(2)
+    assert off.max() <= 6 * np.finfo(float).eps, off.max() / np.finfo(float).eps
