@@ -15,8 +15,8 @@
 // iterations and 3.3 ms, against 180 and 30.4 ms on the curl-curl system with
 // its vectors in memory.
 //
-// Cells whose A^-1 is not positive definite or not finite, or whose contrast
-// exceeds kMaxContrast, are flagged and left to the curl-curl solver.
+// Cells whose A^-1 is not positive definite or not finite, or varies by more than
+// kMaxContrast, are flagged and left to the curl-curl solver.
 #include "msfec_rt3_proj.hpp"
 
 #include "msfec.h"
@@ -35,12 +35,17 @@ using msfec_wave::waves_sum;
 using namespace msfec_trig;
 
 constexpr double kGp[2] = {0.21132486540518711775, 0.78867513459481288225};
-// Largest ratio of the eigenvalue bounds (for an isotropic A^-1 6.75 times its
-// contrast) that is solved here.  Iterations grow with the square root of the
-// contrast, those of the curl-curl solver hardly: 8 cells of 16^3 with
-// lognormal A^-1 of contrast 2.8e3 take 4.5 ms here and 8.6 ms there, of
-// contrast 2.7e5 14.3 ms and 10.4 ms; 27 cells of 8^3 0.5 and 2.3 ms, 1.1 and
-// 3.1 ms.
+// Largest ratio that is solved here of the bounds of the eigenvalues of A^-1 in a
+// cell: the largest trace over the smallest 4 det / trace^2, for isotropic
+// tensors 6.75 times their contrast.  Iterations grow with its square root, those
+// of the curl-curl solver hardly.  Batches on one side alone, 8 cells with
+// lognormal A^-1, here and there: 16^3 at a ratio of 1e4 4.2 and 12 ms, 3e5 12
+// and 17, 1e7 40 and 22; 8^3 at 1e5 1.0 and 4.8 ms, 1e6 2.5 and 6.8, 2e7 6.1 and
+// 7.2; 4^3 at 1e7 0.6 and 1.7 ms.  They cross at about 2e6 (16^3) and 5e7 (8^3).
+// The line is lower because a batch with cells on both sides of it runs both
+// solvers, one after the other: 8 cells of 16^3 with ratios of 6e4 to 2e5 take
+// 16.7 ms, 13.3 with the curl-curl solver alone; at 1e6 the first half of such a
+// batch would add 13 ms to the second.
 constexpr double kMaxContrast = 1e5;
 
 template <int M>
@@ -141,8 +146,9 @@ __global__ __launch_bounds__(Cfg<M>::CT) void rt3_proj_mass_kernel(Rt3Proj g) {
 typedef unsigned mass_v4 __attribute__((ext_vector_type(4)));
 
 // One face basis of one coarse cell per workgroup; a thread owns LZ fine cells
-// of a column in z and the lower face of each of them in every direction (x, r
-// and p of these in registers).  M_A p cell by cell: the upper faces of a cell
+// of a column in z and the lower face of each of them in every direction (r and p
+// of these in registers, as far as they go: 336 bytes a lane of the kernel for
+// M = 16 are in scratch; x in the output buffer).  M_A p cell by cell: the upper faces of a cell
 // belong to its neighbours, whose p come, and to whom the products go, by lane
 // shifts along x, through LDS along y and in the column along z.  Then r goes
 // to the lattice E in LDS, which the transforms turn into z.
