@@ -36,10 +36,11 @@ FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X FP32 matrix cores, dense
 # it and reported with their ratio to it.
 SOLVERS = {"band-fp64-mfma": (1, "q_blk_factor_kernel<double>", "f64"),
            "band-mixed": (2, "q_blk_factor_kernel<float>", "f32"),
-           "band-fp64-valu": (0, "q_band_kernel", "f64")}
+           "band-fp64": (0, "q_blk_factor_kernel<double>", "f64")}
 SOLVER_TEXT = {"band-mixed": "banded Cholesky FP32 on the matrix cores + iterative refinement "
                              "with FP64 residuals until (|dx|/|x|)^2 <= 1e-11 per cell",
-               "band-fp64-valu": "banded Cholesky FP64 on the vector ALUs",
+               "band-fp64": "banded Cholesky FP64 on the matrix cores, LDL^T on the vector "
+                            "ALUs for the cells that are not positive definite",
                "band-fp64-mfma": "banded Cholesky FP64 on the matrix cores"}
 HEADLINE = "band-fp64-mfma"
 TRAFFIC_FILE = os.path.join(REPO, "profiles", "hbm_traffic.json")

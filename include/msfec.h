@@ -114,10 +114,10 @@ typedef struct {
   int max_refine;      /* BAND_MIXED: refinement steps at most (0 = 3)     */
   double cg_tol;       /* CG: relative residual to reach (0 = 1e-13)       */
   int cg_max_iter;     /* CG: iterations at most (0 = 5000)                */
-  int band_window;     /* BAND_FP64_MFMA, scalar coefficient: slots of the
-                          band window, 16, 32 or 64 (it must hold the
-                          half-bandwidth + 4); 0 = the smallest that does.
-                          The other solvers keep 64.                       */
+  int band_window;     /* BAND_FP64_MFMA and BAND_FP64, scalar coefficient:
+                          slots of the matrix-core band window, 16, 32 or 64
+                          (it must hold the half-bandwidth + 4); 0 = the
+                          smallest that does.  The other solvers keep 64.  */
 } msfec_q_params;
 
 typedef struct {
@@ -275,8 +275,8 @@ msfec_status msfec_q_adjoint_gradient(msfec_q_handle h, int nc, const double *u_
  * local solver:
  *   - solver MSFEC_SOLVER_AUTO: where the interior band fits the band window
  *     (3-D l <= 3, 2-D l <= 5) the fastest of the FP64 solvers and tile
- *     shapes (matrix-core band with a 16-, 32- or 64-slot window, vector-ALU
- *     band, CG), timed on up to 256 of the level's own cells
+ *     shapes (matrix-core band with a 16-, 32- or 64-slot window; BAND_FP64
+ *     where these fail; CG), timed on up to 256 of the level's own cells
  *     with the current coefficients (a candidate whose cells do not all come
  *     out MSFEC_CELL_OK is rejected); matrix-free CG beyond the window.  The
  *     choice is made by msfec_qu_tune, or by the first compute when no tuning
@@ -320,7 +320,7 @@ msfec_status msfec_qu_tune(msfec_qu_handle h);
 /* The solver of a level present in the batch, its band window (slots; 0
  * for the solvers without one), its cell count and, when tuned, the timed
  * milliseconds of the 5 candidates (matrix-core band with a 16-, 32- and
- * 64-slot window, vector-ALU band, CG; -1 where not timed, not applicable or
+ * 64-slot window, BAND_FP64, CG; -1 where not timed, not applicable or
  * rejected).  Any pointer may be NULL. */
 msfec_status msfec_qu_level_info(msfec_qu_handle h, int level, int *solver, int *window,
                                  int *n_cells, float *ms5);

@@ -4626,7 +4626,8 @@ msfec_status msfec_q_create(const msfec_q_params* params, int n_cells, const dou
   fill_qconf(p, c);
   h->fast = (p.coef_mode == MSFEC_COEF_SCALAR_CELL) && (p.rhs_mode != MSFEC_RHS_QP);
   // the mixed solver's refinement sweep and the general path keep the 64-slot window
-  c.nt = (p.solver == MSFEC_SOLVER_BAND_FP64_MFMA && h->fast) ? band_tile_rows(bw, p.band_window) : 4;
+  const bool f64 = p.solver == MSFEC_SOLVER_BAND_FP64_MFMA || p.solver == MSFEC_SOLVER_BAND_FP64;
+  c.nt = (f64 && h->fast) ? band_tile_rows(bw, p.band_window) : 4;
   const int nq = nv;
   h->coef_count = (p.coef_mode == MSFEC_COEF_SCALAR_CELL)
                       ? (size_t)n_cells * c.nfc
@@ -4992,7 +4993,7 @@ msfec_status msfec_q_compute(msfec_q_handle h, void* stream) {
     // the non-finite values came first.  For all cells that kernel takes twice
     // the time at every size (a pass of 125 cells of 8^3 458 against 230 us, of
     // 4096 1775 and 904; 64 of 32^2 1130 and 552, 1024 of 2^2 62 and 47).
-    if (fast) launch_factor64(c.dim, mfma ? c.nt : band_tile_rows(h->bw, h->p.band_window), h->n_cells, s, a);
+    if (fast) launch_factor64(c.dim, c.nt, h->n_cells, s, a);
     else if (c.dim == 3) LAUNCH_BAND(q_band_mfma_kernel, 3, false);
     else LAUNCH_BAND(q_band_mfma_kernel, 2, false);
     if (!mfma) {

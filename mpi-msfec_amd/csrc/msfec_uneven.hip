@@ -82,7 +82,8 @@ int ipow_qu(int b, int e) {
 
 // candidates timed for a level inside the band window, in tie-break order:
 // the matrix-core band with a 16-, 32- and 64-slot window (the tile shape:
-// 1, 2 or 4 tile rows of 16), the vector-ALU band, CG
+// 1, 2 or 4 tile rows of 16); BAND_FP64 where none of these succeeds (where one
+// does it is the same kernel and a launch more); CG
 struct Cand {
   int solver, window;
 };
@@ -263,6 +264,8 @@ msfec_status qu_tune(msfec_qu_batch* h) {
     }
     int best = -1;
     for (int k = 0; k < kNCand; ++k) {
+      L.ms[k] = -1.f;
+      if (kCand[k].solver == MSFEC_SOLVER_BAND_FP64 && best >= 0) continue;
       QU_TRY(time_candidate(h, L, kCand[k], &L.ms[k]));
       if (L.ms[k] >= 0.f && (best < 0 || L.ms[k] < L.ms[best])) best = k;
     }

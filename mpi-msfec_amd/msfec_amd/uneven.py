@@ -23,11 +23,11 @@ import numpy as np
 from . import _lib as L
 from .qbasis import _ptr
 
-SOLVER_NAMES = {L.SOLVER_BAND_FP64: "band-fp64-valu", L.SOLVER_BAND_FP64_MFMA: "band-fp64-mfma",
+SOLVER_NAMES = {L.SOLVER_BAND_FP64: "band-fp64", L.SOLVER_BAND_FP64_MFMA: "band-fp64-mfma",
                 L.SOLVER_BAND_MIXED: "band-mixed", L.SOLVER_CG: "cg"}
 #: the timed candidates of a level (solver and band window), in the order
 #: msfec_qu_level_info reports them
-CANDIDATES = ("band_mfma_w16", "band_mfma_w32", "band_mfma_w64", "band_valu", "cg")
+CANDIDATES = ("band_mfma_w16", "band_mfma_w32", "band_mfma_w64", "band_fp64", "cg")
 
 
 def band_fits(dim: int, level: int) -> bool:

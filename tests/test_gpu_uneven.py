@@ -173,3 +173,24 @@ def test_uneven_device_buffers_match_host():
                 x.free()
     for x, y, name in zip(got, (M, b, P), ("M", "b", "Psi")):
         np.testing.assert_array_equal(x, y, err_msg=name)
+
+
+def test_tuner_times_no_kernel_twice():
+    """BAND_FP64 starts with the matrix-core kernel: it is a candidate only
+    where that one fails with every window, and its batch reports the same
+    window."""
+    print("case uneven tuner candidates", flush=True)
+    from msfec_amd import QBasisBatch, UnevenBatch, _lib as L, fields as F
+    verts = F.coarse_vertices(3, 2)
+    lv = np.array([1, 2, 3, 1, 2, 3, 1, 2])
+    blocks = [np.ones(8 ** l) for l in lv]
+    with UnevenBatch(verts, lv, dim=3, coef_blocks=blocks) as ub:
+        ub.tune()
+        for l, s in ub.summary().items():
+            assert s["tuned_ms"]["band_fp64"] is None and s["tuned_ms"]["cg"] is not None
+            assert s["solver"] in ("band-fp64-mfma", "cg")
+    for dim, l, window in ((2, 3, 16), (3, 2, 32), (3, 3, 64)):
+        for solver in (L.SOLVER_BAND_FP64, L.SOLVER_BAND_FP64_MFMA):
+            with QBasisBatch(F.coarse_vertices(dim, 1), dim=dim, n_refine_local=l,
+                             solver=solver) as qb:
+                assert qb.info.band_window == window
