@@ -4993,6 +4993,10 @@ msfec_status msfec_q_compute(msfec_q_handle h, void* stream) {
     // the non-finite values came first.  For all cells that kernel takes twice
     // the time at every size (a pass of 125 cells of 8^3 458 against 230 us, of
     // 4096 1775 and 904; 64 of 32^2 1130 and 552, 1024 of 2^2 62 and 47).
+    // Cells that are not positive definite take both, one after the other: 64 of
+    // 8^3 with a reaction rate of -800 per cell 603 us, 416 by the one-pivot
+    // kernel alone.  Leaving the first kernel at a bad pivot made that 444 to 522
+    // us, and every other pass 0.6 to 1.2 % slower.
     if (fast) launch_factor64(c.dim, c.nt, h->n_cells, s, a);
     else if (c.dim == 3) LAUNCH_BAND(q_band_mfma_kernel, 3, false);
     else LAUNCH_BAND(q_band_mfma_kernel, 2, false);
