@@ -25,6 +25,7 @@
 #include "msfec_lines.hpp"
 
 #include "msfec.h"
+#include "msfec_wave.hpp"
 
 namespace {
 
@@ -43,15 +44,6 @@ struct Lines {
   static constexpr int WL = ND * 256, WR = WL + TB * 256, WF = WR + TB * 256, LINE = WF + TT * 128;
 };
 
-__device__ __forceinline__ double inv_sqrt(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  y = y * fma(-0.5 * x * y, y, 1.5);
-  return y * fma(-0.5 * x * y, y, 1.5);
-}
-__device__ __forceinline__ double lane_of(double v, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                          __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
 // lane K of each row of 16 lanes, in all of them
 template <int K>
 __device__ __forceinline__ double row_lane(double v) {
@@ -79,9 +71,9 @@ template <int K>
 __device__ __forceinline__ void chol_step(v4& z, int lane, bool& ok) {
   constexpr int R = K / 4, H = K % 4;
   const int lh = lane >> 4, ll = lane & 15;
-  const double piv = lane_of(z[R], 16 * H + K);
+  const double piv = msfec_wave::lane_value(z[R], 16 * H + K);
   ok = ok && piv > 0.0 && piv < INFINITY;
-  const double rs = inv_sqrt(piv);
+  const double rs = msfec_wave::inv_sqrt(piv);
   const int from = (16 * H + ll) * 4;
   double row = __hiloint2double(__builtin_amdgcn_ds_bpermute(from, __double2hiint(z[R])),
                                 __builtin_amdgcn_ds_bpermute(from, __double2loint(z[R])));

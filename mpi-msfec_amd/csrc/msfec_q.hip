@@ -1802,14 +1802,9 @@ __device__ __forceinline__ float bk_readlane(float v, int l) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 
-// 1/sqrt: the hardware estimate, refined by two Newton steps in FP64 (one
-// step is not enough for FP64; the FP32 estimate is already within 1 ulp).
-__device__ __forceinline__ double bk_rsqrt(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  y = y * fma(-0.5 * x * y, y, 1.5);
-  y = y * fma(-0.5 * x * y, y, 1.5);
-  return y;
-}
+// 1/sqrt: in FP64 the hardware estimate refined by two Newton steps (one is not
+// enough); the FP32 estimate is already within 1 ulp.
+__device__ __forceinline__ double bk_rsqrt(double x) { return msfec_wave::inv_sqrt(x); }
 __device__ __forceinline__ float bk_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
 
 // Pivot monitor: the smallest pivot (NaN ignored) and the sum of all pivots.

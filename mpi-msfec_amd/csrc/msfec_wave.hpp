@@ -1,4 +1,4 @@
-// Buffer loads, lane shifts, and sums over a wave and a workgroup.
+// Buffer loads, lane shifts, sums over a wave and a workgroup, the inverse root.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -56,6 +56,17 @@ template <int NW>
 __device__ __forceinline__ double waves_sum(const double* red) {
   static_assert(NW <= 16, "one row");
   return row_sum<NW>(red[threadIdx.x & (NW - 1)]);
+}
+
+// x^-1/2 for x > 0: the instruction and two Newton steps, the last one as a
+// correction of the value, which leaves about one rounding (y (1.5 - x y^2 / 2)
+// leaves three: the bases of the band solver were off by 1.04e-15 to 1.91e-14
+// instead of 8.6e-16 to 1.58e-14 then, 5 % to 20 % more than with divisions; a
+// step takes as long)
+__device__ __forceinline__ double inv_sqrt(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  y = y * fma(-0.5 * x * y, y, 1.5);
+  return fma(0.5 * y, fma(-x * y, y, 1.0), y);
 }
 
 // v of the lane to the right (left); zero at the ends of a row of 16 lanes
