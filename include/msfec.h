@@ -611,8 +611,9 @@ typedef struct {
   int n_refine_local; /* l, 1..4                                                  */
   int flags;          /* MSFEC_FLAG_*                                             */
   int max_iter;       /* CG iteration limit, 0: 20000 (MSFEC_CELL_NOT_CONVERGED) */
-  double rtol;        /* CG stop: preconditioned residual (curl-curl: residual) <=
-                         rtol x the initial one, 0: 1e-13                        */
+  double rtol;        /* CG stop: residual <= rtol x the initial one on the
+                         curl-curl system, preconditioned residual <= rtol / 2 x
+                         the initial one on the fluxes; 0: 1e-13                 */
 } msfec_rt3_params;
 
 typedef struct msfec_rt3_batch *msfec_rt3_handle;

@@ -134,3 +134,31 @@ def test_balance_of_every_fine_cell(l, dev):
     want = np.array([-1.0, 1, -1, 1, -1, 1])[None, :, None, None, None] / m ** 3
     off = np.abs(x + y + z - want).max((2, 3, 4)) / np.abs(S).max(2)
     assert off.max() <= 6 * np.finfo(float).eps, off.max() / np.finfo(float).eps
+
+
+def test_default_stop(oracle_mod):
+    """8 cells of 8^3 with the oscillatory tensor of the reference example: the
+    mean error of the fluxes at the default rtol is at most what the curl-curl
+    solver's |r| <= 1e-13 |b| leaves there (1.7e-14 in the 2-norm; the oracle
+    is refined to rounding)."""
+    print("case rt3 default stop", flush=True)
+    from msfec_amd import fields as F
+    l, N, n = 3, 8, 8
+    verts = F.coarse_vertices(3, 2)
+    i = np.arange(N ** 3)
+    cell = np.stack([i % N, i // N % N, i // (N * N)], -1)
+    q = np.arange(8)
+    gp = np.array([0.5 - 0.5 / np.sqrt(3), 0.5 + 0.5 / np.sqrt(3)])
+    pt = (cell[:, None] + gp[np.stack([q & 1, q >> 1 & 1, q >> 2], -1)]) / N
+    x = verts[:, 0][:, None, None] + pt * 0.5
+    phase = np.array([0.1, 0.45, 0.8])
+    d = 1.0 / (1.0 - 0.9 * np.sin(2 * np.pi * (np.array([17.0, 16.0, 15.0]) * x + phase)))
+    R = F._euler_rotation()
+    ainv = np.stack([(R[a] * R[b] * d).sum(-1)
+                     for a, b in ((0, 0), (0, 1), (0, 2), (1, 1), (1, 2), (2, 2))], -1)
+    _, _, S, st, its = run(verts, l, ainv)
+    assert (st == 0).all()
+    e = [np.linalg.norm(S[c] - So) / np.linalg.norm(So)
+         for c in range(n) for So in [oracle_mod.rt3_basis_cell(l, verts[c], ainv[c], None)[2]]]
+    print("mean %.2e max %.2e its %d" % (np.mean(e), np.max(e), its.max()), flush=True)
+    assert np.mean(e) <= 1.7e-14
