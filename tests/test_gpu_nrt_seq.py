@@ -45,19 +45,25 @@ def test_matches_oracle(oracle_mod, l, n, load):
 
 
 def test_l4_matches_minres():
-    """Two cells of 16^3 against MINRES on the full system, which stops at
-    1e-14 of its residual (1e-8 on the bases, the tolerance of its tests)."""
+    """Two cells of 16^3 against MINRES on the full system.  Element matrix and
+    load are of second order in the error of either: 1e-12 (2e-15 and 4e-14
+    measured).  The bases of MINRES itself are off by up to 1e-9 here (2e-10 to
+    4e-10 between its rtol of 1e-14 and 1e-16): 1e-8, the tolerance of its
+    tests; those of the sequence must stay within 1e-12 when its rtol goes from
+    1e-14 to 1e-17 (3e-14 measured)."""
     print("case nrt sequence l=4", flush=True)
     from msfec_amd import _lib as L
     rng = np.random.default_rng(3104)
     verts = boxes(rng, 2)
     ainv, bq, _, fq = rand_coefs(rng, 2, 4, reaction=False)
     a = run(verts, 4, ainv, bq, None, fq)
+    t = run(verts, 4, ainv, bq, None, fq, rtol=1e-17)
     g = run(verts, 4, ainv, bq, None, fq, solver=L.SOLVER_CG)
-    assert (a[3] == 0).all() and (g[3] == 0).all()
+    assert (a[3] == 0).all() and (t[3] == 0).all() and (g[3] == 0).all()
     for c in range(2):
-        assert rel(a[0][c], g[0][c]) <= 1e-8 and rel(a[1][c], g[1][c]) <= 1e-8
+        assert rel(a[0][c], g[0][c]) <= 1e-12 and rel(a[1][c], g[1][c]) <= 1e-12
         assert max(rel(a[2][c, i], g[2][c, i]) for i in range(18)) <= 1e-8
+        assert max(rel(a[2][c, i], t[2][c, i]) for i in range(18)) <= 1e-12
 
 
 @pytest.mark.parametrize("l", [1, 2, 3])
