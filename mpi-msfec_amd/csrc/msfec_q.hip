@@ -3868,8 +3868,8 @@ __global__ __launch_bounds__(64 * kFinWaves) void q_cg_finish_kernel(BandArgs a,
 }
 
 // ---------------------------------------------------------------------------
-// CG on the assembled stencil: tensor coefficients at the Gauss points and /
-// or loads per Gauss point (the reference's Diffusion_A and
+// CG on the assembled stencil in 2-D: tensor coefficients at the Gauss points
+// and / or loads per Gauss point (the reference's Diffusion_A and
 // RightHandSideParsed evaluated at the QGauss(2) points, q_basis.cc:196-220),
 // solved matrix-free beyond the band window.  q_assemble_kernel has written
 // the lower stencil Slo of every node (diagonal first, then the lower
@@ -3880,10 +3880,9 @@ __global__ __launch_bounds__(64 * kFinWaves) void q_cg_finish_kernel(BandArgs a,
 // Slo[n][0] p[n] + sum_t Slo[n][t] p[n - off_t] + Slo[n + off_t][t] p[n + off_t]
 // with the stencil rows read from global memory (L2) each iteration.
 // ---------------------------------------------------------------------------
-template <int DIM>
 __device__ __forceinline__ double cg_stencil_row(const double* __restrict__ slo, const int* off,
                                                  int node, const double* v) {
-  using D = Dirs<DIM>;
+  using D = Dirs<2>;
   double acc = slo[(size_t)node * D::NLOW] * v[node];
 #pragma unroll
   for (int t = 1; t < D::NLOW; ++t) {
@@ -3894,9 +3893,8 @@ __device__ __forceinline__ double cg_stencil_row(const double* __restrict__ slo,
   return acc;
 }
 
-template <int DIM>
 __global__ __launch_bounds__(kCgThreads) void q_cg_stencil_kernel(BandArgs a, CgArgs g, QConf c) {
-  using D = Dirs<DIM>;
+  using D = Dirs<2>;
   const int cell = blockIdx.x / g.nsolve, j = blockIdx.x - cell * g.nsolve;
   const int tid = threadIdx.x;
   extern __shared__ double dyn[];  // search direction over all nodes
@@ -3907,13 +3905,13 @@ __global__ __launch_bounds__(kCgThreads) void q_cg_stencil_kernel(BandArgs a, Cg
   for (int z = tid; z < a.nn; z += kCgThreads) pv[z] = 0.0;
   const double* slo = a.Slo + (size_t)cell * a.nn * D::NLOW;
   const int ni = a.ni, L = g.seg, spl = (ni + L - 1) / L;
-  const int lines = (DIM == 3) ? ni * ni : ni;
+  const int lines = ni;
   const int line0 = tid / spl, sx = tid - line0 * spl;
   const int len = (line0 < lines) ? min(L, ni - sx * L) : 0;
   const int line = (line0 < lines) ? line0 : 0;
-  const int x0 = 1 + sx * L, cy = 1 + line % ni, cz = (DIM == 3) ? 1 + line / ni : 0;
-  const int jn0 = (x0 - 1) + ni * ((cy - 1) + (DIM == 3 ? ni * (cz - 1) : 0));
-  const int node0 = x0 + a.S * cy + (DIM == 3 ? a.S * a.S * cz : 0);
+  const int x0 = 1 + sx * L, cy = 1 + line;
+  const int jn0 = (x0 - 1) + ni * (cy - 1);
+  const int node0 = x0 + a.S * cy;
   double b[kCgOwn], dinv[kCgOwn], x[kCgOwn], r[kCgOwn], p[kCgOwn];
   double bb = 0.0, rz = 0.0;
 #pragma unroll
@@ -3942,7 +3940,7 @@ __global__ __launch_bounds__(kCgThreads) void q_cg_stencil_kernel(BandArgs a, Cg
     }
     double q[kCgOwn];
 #pragma unroll
-    for (int t = 0; t < kCgOwn; ++t) q[t] = (t < len) ? cg_stencil_row<DIM>(slo, off, node0 + t, pv) : 0.0;
+    for (int t = 0; t < kCgOwn; ++t) q[t] = (t < len) ? cg_stencil_row(slo, off, node0 + t, pv) : 0.0;
     double pq = 0.0;
 #pragma unroll
     for (int t = 0; t < kCgOwn; ++t)
@@ -3991,7 +3989,7 @@ __global__ __launch_bounds__(kCgThreads) void q_cg_stencil_kernel(BandArgs a, Cg
     if (t < len) {
       const size_t jn = (size_t)cell * a.n + jn0 + t;
       a.X[jn * kMaxNb + j] = x[t];
-      a.Rres[jn * kMaxNb + j] = b[t] - cg_stencil_row<DIM>(slo, off, node0 + t, pv);
+      a.Rres[jn * kMaxNb + j] = b[t] - cg_stencil_row(slo, off, node0 + t, pv);
       psi[node0 + t] = x[t];
     }
   }
@@ -4007,18 +4005,15 @@ __global__ __launch_bounds__(kCgThreads) void q_cg_stencil_kernel(BandArgs a, Cg
 // the interior solution: psi_k is K-harmonic at the interior rows and the
 // error vanishes on the boundary.  Psi is completed on the boundary with the
 // lifted coarse shape functions first; then every thread takes every 512th
-// node, forms (K psi_k)(node) for the 2^dim bases and accumulates the 64
-// products and the 8 loads, summed over the workgroup at the end.  512
-// threads: the 72 accumulators need more than the 128 registers a thread of
-// a 1024-thread workgroup may hold.
+// node, forms (K psi_k)(node) for the 4 bases and accumulates the 16 products
+// and the 4 loads, summed over the workgroup at the end.
 constexpr int kTfThreads = 512;
 
-template <int DIM>
 __global__ __launch_bounds__(kTfThreads) void q_cg_tensor_finish_kernel(BandArgs a, CgArgs g,
                                                                         QConf c) {
-  using D = Dirs<DIM>;
+  using D = Dirs<2>;
   const int cell = blockIdx.x, tid = threadIdx.x;
-  __shared__ double part[kTfThreads / 64][72];
+  __shared__ double part[kTfThreads / 64][D::NV * D::NV + D::NV];
   __shared__ int off[D::NLOW];
   if (tid < D::NLOW) off[tid] = c.off_full[tid];
   double* psi = a.Psi + (size_t)cell * D::NV * a.nn;
@@ -4028,7 +4023,7 @@ __global__ __launch_bounds__(kTfThreads) void q_cg_tensor_finish_kernel(BandArgs
     int m[3] = {0, 0, 0}, rr = node;
     bool bnd = false;
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) {
+    for (int d = 0; d < 2; ++d) {
       m[d] = rr % a.S;
       rr /= a.S;
       bnd = bnd || m[d] == 0 || m[d] == a.N;
@@ -4046,14 +4041,14 @@ __global__ __launch_bounds__(kTfThreads) void q_cg_tensor_finish_kernel(BandArgs
   for (int node = tid; node < a.nn; node += kTfThreads) {
     int m[3] = {0, 0, 0}, rr = node;
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) {
+    for (int d = 0; d < 2; ++d) {
       m[d] = rr % a.S;
       rr /= a.S;
     }
     double kp[D::NV];
 #pragma unroll
     for (int k = 0; k < D::NV; ++k) kp[k] = slo[(size_t)node * D::NLOW] * psi[(size_t)k * a.nn + node];
-    // the 3^dim - 1 neighbours inside the grid: lower ones from the own row,
+    // the 8 neighbours inside the grid: lower ones from the own row,
     // upper ones from the neighbour's row
 #pragma unroll
     for (int t = 1; t < D::NLOW; ++t) {
@@ -4062,7 +4057,7 @@ __global__ __launch_bounds__(kTfThreads) void q_cg_tensor_finish_kernel(BandArgs
       bool lo_ok = true, up_ok = true;
       int ee = e;
 #pragma unroll
-      for (int d = 0; d < DIM; ++d) {
+      for (int d = 0; d < 2; ++d) {
         const int dd = ee % 3 - 1;  // offset of the lower neighbour in direction d is dd
         ee /= 3;
         if (m[d] + dd < 0 || m[d] + dd > a.N) lo_ok = false;
@@ -4897,15 +4892,9 @@ msfec_status msfec_q_compute(msfec_q_handle h, void* stream) {
     const bool reac = c.reaction_mode != MSFEC_REACTION_NONE;
     g.nsolve = reac ? c.nv : c.nv - 1;
     const size_t cdyn = (size_t)c.nn * sizeof(double);
-#define LAUNCH_CGS(D)                                                                     \
-  do {                                                                                    \
-    MSFEC_HIP(hipFuncSetAttribute((const void*)q_cg_stencil_kernel<D>,                    \
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)cdyn)); \
-    hipLaunchKernelGGL((q_cg_stencil_kernel<D>), dim3(h->n_cells * g.nsolve), dim3(kCgThreads), \
-                       cdyn, s, a, g, c);                                                 \
-  } while (0)
-    LAUNCH_CGS(2);
-#undef LAUNCH_CGS
+    MSFEC_HIP(hipFuncSetAttribute((const void*)q_cg_stencil_kernel,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)cdyn));
+    hipLaunchKernelGGL(q_cg_stencil_kernel, dim3(h->n_cells * g.nsolve), dim3(kCgThreads), cdyn, s, a, g, c);
     MSFEC_HIP(hipGetLastError());
     if (!reac) {
       const unsigned ub = (unsigned)(((size_t)h->n_cells * c.n + 255) / 256);
@@ -4913,7 +4902,7 @@ msfec_status msfec_q_compute(msfec_q_handle h, void* stream) {
       MSFEC_HIP(hipGetLastError());
     }
     if (tm) MSFEC_HIP(hipEventRecord(ev[2], s));
-    hipLaunchKernelGGL((q_cg_tensor_finish_kernel<2>), dim3(h->n_cells), dim3(kTfThreads), 0, s, a, g, c);
+    hipLaunchKernelGGL(q_cg_tensor_finish_kernel, dim3(h->n_cells), dim3(kTfThreads), 0, s, a, g, c);
     MSFEC_HIP(hipGetLastError());
     if (tm) MSFEC_HIP(hipEventRecord(ev[3], s));
   } else if (h->p.solver == MSFEC_SOLVER_CG) {
