@@ -33,6 +33,7 @@
 #include "msfec_nrt_seq.hpp"
 
 #include "msfec.h"
+#include "msfec_cell.hpp"
 #include "msfec_q1t.hpp"
 #include "msfec_trig.hpp"
 #include "msfec_wave.hpp"
@@ -41,13 +42,9 @@ namespace {
 
 using msfec_detail::NrtSeq;
 using namespace msfec_trig;
+using namespace msfec_cell;
 using msfec_wave::block_sums;
 using msfec_wave::wave_sum;
-
-constexpr double kGp[2] = {0.21132486540518711775, 0.78867513459481288225};
-constexpr int kLnAx[12] = {1, 1, 0, 0, 1, 1, 0, 0, 2, 2, 2, 2};
-constexpr int kLnF1[12] = {0, 1, 0, 1, 0, 1, 0, 1, 0, 1, 0, 1};
-constexpr int kLnF2[12] = {0, 0, 0, 0, 1, 1, 1, 1, 0, 0, 1, 1};
 
 template <int M>
 struct Seq {

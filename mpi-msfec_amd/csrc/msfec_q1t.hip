@@ -3,6 +3,7 @@
 #include "msfec_q1t.hpp"
 
 #include "msfec.h"
+#include "msfec_cell.hpp"
 #include "msfec_wave.hpp"
 
 #include <algorithm>
@@ -12,6 +13,7 @@ namespace {
 using msfec_detail::Q1tBasis;
 using msfec_detail::Q1tCg;
 using msfec_detail::Q1tRows;
+using namespace msfec_cell;
 using msfec_wave::block_sums;
 using msfec_wave::buffer_f64;
 using msfec_wave::buffer_of;
@@ -19,13 +21,6 @@ using msfec_wave::from_left;
 using msfec_wave::from_right;
 using msfec_wave::wave_sum;
 
-constexpr double kGp[2] = {0.21132486540518711775, 0.78867513459481288225};
-
-// deal.II's line order on the unit cube: axis, and the fixed values of the
-// two other coordinates (lower axis first)
-constexpr int kLnAx[12] = {1, 1, 0, 0, 1, 1, 0, 0, 2, 2, 2, 2};
-constexpr int kLnF1[12] = {0, 1, 0, 1, 0, 1, 0, 1, 0, 1, 0, 1};
-constexpr int kLnF2[12] = {0, 0, 0, 0, 1, 1, 1, 1, 0, 0, 1, 1};
 
 // The nodes of one workgroup of the assembly: whole rows in x, TY x TZ of
 // them.  The tensors of the cells around them are staged in LDS two Gauss

@@ -20,12 +20,14 @@
 #include "msfec_rt3_proj.hpp"
 
 #include "msfec.h"
+#include "msfec_cell.hpp"
 #include "msfec_trig.hpp"
 #include "msfec_wave.hpp"
 
 namespace {
 
 using msfec_detail::Rt3Proj;
+using namespace msfec_cell;
 using msfec_wave::block_sums;
 using msfec_wave::buffer_f64;
 using msfec_wave::from_left;
@@ -34,7 +36,6 @@ using msfec_wave::wave_sum;
 using msfec_wave::waves_sum;
 using namespace msfec_trig;
 
-constexpr double kGp[2] = {0.21132486540518711775, 0.78867513459481288225};
 // Largest ratio that is solved here of the bounds of the eigenvalues of A^-1 in a
 // cell: the largest trace over the smallest 4 det / trace^2, for isotropic
 // tensors 6.75 times their contrast.  Iterations grow with its square root, those
