@@ -276,7 +276,7 @@ msfec_status msfec_q_adjoint_gradient(msfec_q_handle h, int nc, const double *u_
  *   - solver MSFEC_SOLVER_AUTO: where the interior band fits the band window
  *     (3-D l <= 3, 2-D l <= 5) the fastest of the FP64 solvers and tile
  *     shapes (matrix-core band with a 16-, 32- or 64-slot window; BAND_FP64
- *     where these fail; CG), timed on up to 256 of the level's own cells
+ *     where these fail; CG), timed on up to 2048 of the level's own cells
  *     with the current coefficients (a candidate whose cells do not all come
  *     out MSFEC_CELL_OK is rejected); matrix-free CG beyond the window.  The
  *     choice is made by msfec_qu_tune, or by the first compute when no tuning

@@ -93,7 +93,12 @@ constexpr Cand kCand[kNCand] = {{MSFEC_SOLVER_BAND_FP64_MFMA, 16},
                                 {MSFEC_SOLVER_BAND_FP64_MFMA, 64},
                                 {MSFEC_SOLVER_BAND_FP64, 0},
                                 {MSFEC_SOLVER_CG, 0}};
-constexpr int kTuneCells = 256;
+// Cells of a level that are timed: as many as the band kernels, one wave a cell and
+// two waves a SIMD, hold on the card at once.  With fewer the band is timed by its
+// latency and CG, seven workgroups a cell, by its throughput.  16^3 cells at levels
+// 2 to 4: 256 cells of level 3 take them 0.21 and 0.20 ms, all 1856 0.39 and 1.22;
+// a pass takes 5.5 ms with the choice from 256 cells and 4.9 ms from these.
+constexpr int kTuneCells = 2048;
 
 struct Level {
   int level = 0;

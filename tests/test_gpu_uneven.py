@@ -194,3 +194,20 @@ def test_tuner_times_no_kernel_twice():
             with QBasisBatch(F.coarse_vertices(dim, 1), dim=dim, n_refine_local=l,
                              solver=solver) as qb:
                 assert qb.info.band_window == window
+
+
+def test_tuner_sample_fills_the_card():
+    """The choice is that of the whole level: 256 cells of 8^3 with a constant
+    coefficient take CG half as long as the band, 1800 a third longer."""
+    print("case uneven tuner sample", flush=True)
+    from msfec_amd import UnevenBatch, fields as F
+    nc = 13
+    n = nc ** 3
+    lv = np.where(np.arange(n) < 1800, 3, 1)
+    blocks = [np.ones(8 ** l) for l in lv]
+    with UnevenBatch(F.coarse_vertices(3, nc), lv, dim=3, coef_blocks=blocks) as ub:
+        ub.tune()
+        s = ub.summary()[3]
+        print(s, flush=True)
+        assert s["solver"] == "band-fp64-mfma"
+        assert s["tuned_ms"]["cg"] > 1.2 * s["tuned_ms"]["band_mfma_w64"]
