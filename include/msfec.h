@@ -613,7 +613,8 @@ typedef struct {
   int max_iter;       /* CG iteration limit, 0: 20000 (MSFEC_CELL_NOT_CONVERGED) */
   double rtol;        /* CG stop: residual <= rtol x the initial one on the
                          curl-curl system, preconditioned residual <= rtol / 2 x
-                         the initial one on the fluxes; 0: 1e-13                 */
+                         the initial one on the fluxes (not below 1e-15 unless
+                         rtol is); 0: 1e-13                                      */
 } msfec_rt3_params;
 
 typedef struct msfec_rt3_batch *msfec_rt3_handle;

@@ -2798,6 +2798,8 @@ msfec_status msfec_nrt_compute(msfec_nrt_handle h, void* stream) {
   // Without a reaction term the exact sequence gives the bases; the general
   // solver then takes the cells that it flags (an indefinite A^-1, B <= 0,
   // data that are not finite) and its workgroups leave the others at once.
+  // (A batch of nothing but such cells pays 25 to 150 us for the attempt: 4096
+  // at l = 1 893 us instead of 813, at l = 2 6.70 ms instead of 6.55.)
   // An explicit MSFEC_SOLVER_CG asks for MINRES.
   const int* need = nullptr;
   if (h->d_seq && !h->has_r) {

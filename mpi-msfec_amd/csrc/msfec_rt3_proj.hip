@@ -354,8 +354,10 @@ __global__ __launch_bounds__(Cfg<M>::NT) void rt3_proj_cg_kernel(Rt3Proj g) {
   }
   // half of rtol: with rtol itself the fluxes were off by up to 1.7 times what
   // |r| <= rtol |b| leaves on the curl-curl system (8^3 cells of the reference
-  // example's tensor 2.8e-14 and 1.7e-14; 1.4e-14 so), for one iteration in 40
-  const double stop = 0.25 * g.rtol * g.rtol * rz;
+  // example's tensor 2.8e-14 and 1.7e-14; 1.4e-14 so), for one iteration in 40.
+  // Not below 1e-15 unless rtol is: rounding need not let it go on.
+  const double tol = fmax(0.5 * g.rtol, fmin(g.rtol, 1e-15));
+  const double stop = tol * tol * rz;
   int it = 0, flag = MSFEC_CELL_OK;
   __syncthreads();
   while (rz > stop) {

@@ -163,3 +163,15 @@ def test_default_stop(oracle_mod):
          for c in range(n) for So in [oracle_mod.rt3_basis_cell(l, verts[c], ainv[c], None)[2]]]
     print("mean %.2e max %.2e its %d" % (np.mean(e), np.max(e), its.max()), flush=True)
     assert np.mean(e) <= 1.7e-14
+
+
+@pytest.mark.parametrize("l", [1, 2, 3])
+def test_smallest_rtol(l):
+    """An rtol of 1e-15 is reached at every size (the stop at half of rtol does
+    not go below what rounding allows)."""
+    print(f"case rt3 smallest rtol l={l}", flush=True)
+    rng = np.random.default_rng(5500 + l)
+    n = 9
+    ainv, _, _, _ = rand_coefs(rng, n, l, reaction=False, load=False)
+    _, _, _, st, its = run(boxes(rng, n), l, ainv, rtol=1e-15, max_iter=1000)
+    assert (st == 0).all(), (st, its.max())
